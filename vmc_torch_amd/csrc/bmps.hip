@@ -21,9 +21,9 @@
 //   and B'_{Ly-1} = C.
 // The tensors are Z2-graded, so rho is block diagonal in the parity of
 // (k, v) (par(k) from the sector each kept eigenvector came from); each
-// block is diagonalised by cyclic two-sided Jacobi in LDS (parallel
-// round-robin ordering, every rotation of a round applied at once as 2 x 2
-// block updates J^T rho J).  Norms are carried as FP64 log scales.
+// block is diagonalised by one-sided Jacobi on its pivoted Cholesky factor,
+// in the registers of one wave (bm_jacobi_wave; blocks above 32: two-sided
+// Jacobi in LDS, bm_jacobi).  Norms are carried as FP64 log scales.
 //
 // One workgroup of 256 threads per (configuration, side); the Grams and the
 // boundary tensors live in a per-slot workspace in HBM, the 64 x 64 working
@@ -157,6 +157,7 @@ struct BmShT {
   int bd[BMAX_LY + 1], nbd[BMAX_LY + 1];
   uint64_t bpm[BMAX_LY + 1], npm[BMAX_LY + 1];   // bond parity masks
   double red[BT / 64];
+  double lam[NB];           // eigenvalues by column of T
   int sec[4];               // m0, m1, n0, n1
   int rot;
 };
@@ -215,6 +216,256 @@ __device__ void bm_mm(int n, int m, int K, const double *X, const double *Y, dou
 #pragma unroll
     for (int b = 0; b < TS; ++b)
       if (i0 + a < n && j0 + b < m) out[(i0 + a) * LD + j0 + b] = acc[a][b];
+}
+
+// -------------------------------------------------- one-sided Jacobi in registers
+// x of lane (l ^ M) within a 16-lane row, by data-parallel primitives (no LDS):
+// quad permutes for 1 and 2, half-mirror (^7) after a quad mirror (^3) for 4,
+// a rotation by 8 for 8.
+template <int M>
+__device__ __forceinline__ int bm_xor32(int v) {
+  if constexpr (M == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);
+  if constexpr (M == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);
+  if constexpr (M == 4)
+    return __builtin_amdgcn_mov_dpp(__builtin_amdgcn_mov_dpp(v, 0x1B, 0xF, 0xF, true), 0x141, 0xF,
+                                    0xF, true);
+  return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);
+}
+template <int M>
+__device__ __forceinline__ double bm_xor(double x) {
+  return __hiloint2double(bm_xor32<M>(__double2hiint(x)), bm_xor32<M>(__double2loint(x)));
+}
+// sum of x over lanes l and l ^ 16 (M = 16) or l ^ 32 (M = 32): the row and half
+// swaps of gfx950; both lanes get the same bits
+template <int M>
+__device__ __forceinline__ double bm_swap_sum(double x) {
+  const unsigned lo = (unsigned)__double2loint(x), hi = (unsigned)__double2hiint(x);
+  if constexpr (M == 16) {
+    const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+  } else {
+    const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+  }
+}
+
+// 1 / sqrt(x): hardware estimate and one cubically convergent step
+__device__ __forceinline__ double bm_rsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(0.375, e, 0.5), y);
+}
+
+// Eigenvectors of a symmetric positive semidefinite m x m block (rows and columns
+// off .. off + m of the upper triangle in R, scaled to a largest diagonal entry of 1,
+// m <= 4 RPL): pivoted Cholesky L L^T = block, then one-sided Jacobi on the columns of
+// L (Veselic and Hari, Numer. Math. 56, 1989): they are rotated in pairs until they are
+// orthogonal; their squared norms are then the eigenvalues and the normalised columns
+// the eigenvectors (no matrix of rotations is kept).  The pivoted factor is close to
+// orthogonal columns already: 5.5 sweeps on average for the 16 x 16 blocks of a 6x6
+// D = 4 chi = 8 boundary, against 13 for the columns of the block itself (half of them
+// rounding noise of a rank-deficient block) and 9 for two-sided Jacobi.
+// One wave holds the block in registers: lane (row group, j) has RPL rows of the two
+// columns t and b of pair j, JB bits of j, four row groups; with JB = 3 a wave works
+// on two blocks at once (lanes 32 .. 63: off, m of the second).  A sweep meets every
+// pair of columns once: with groups of G lanes, the columns b visit the group's lanes
+// in Gray-code order (G rounds, one cross-lane exchange by a single bit per round),
+// then the t columns of a group pair up among themselves in one half of its lanes and
+// the b columns in the other, and G halves.
+//
+// What bounds it: instruction issue of the one wave (about 80 per round, all vector
+// ALU; the rotations are found redundantly in every row group, so nothing waits on
+// LDS or a barrier).  The angle is found in FP32 from the FP64 sums (an angle off by
+// 1e-7 leaves 1e-7 of the pair's product for the next sweep); its cosine and sine are
+// orthonormal to FP64.  Measured on 6x6 D = 4 chi = 8, per 32 x 32 eigensolve with four
+// workgroups on a CU: 80 k cycles; 198 k on the columns of the block itself, and 1754 us
+// per launch of 2048 workgroups with two-sided Jacobi in LDS against 1020 us with this.
+// Columns are orthogonal to 4e-15 of their own norms; eigenvalues
+// below 1e-18 of the largest diagonal entry come out as zero vectors.
+// row: LDS scratch of 4 RPL doubles per block.
+// Output, compacted: columns off .. off + m of T (rows off .. off + m) and lam; the
+// caller has zeroed both.
+template <int JB, int RPL>
+__device__ __forceinline__ void bm_jacobi_wave(const double *R, int ld, int off, int m, int mmax, double *row,
+                               double *T, double *lam) {
+  constexpr int NJ = 1 << JB;   // columns j and j + NJ
+  const int lane = threadIdx.x & 63;
+  const int j = lane & (NJ - 1), rg = (lane >> JB) & 3;
+  double t[RPL] = {}, b[RPL] = {};
+  int rank = 0;
+  {
+    // pivoted Cholesky, the remaining block at and ab, its diagonal at the two columns
+    // in dt, db of every row group; the pivot row goes through LDS (same wave: in order)
+    double at[RPL], ab[RPL];
+    const int c0 = j, c1 = j + NJ;
+#pragma unroll
+    for (int k = 0; k < RPL; ++k) {
+      const int r = rg * RPL + k;
+      at[k] = (r < m && c0 < m) ? R[(off + (r < c0 ? r : c0)) * ld + off + (r < c0 ? c0 : r)]
+                                : 0.0;
+      ab[k] = (r < m && c1 < m) ? R[(off + (r < c1 ? r : c1)) * ld + off + (r < c1 ? c1 : r)]
+                                : 0.0;
+    }
+    double dt = c0 < m ? R[(off + c0) * (ld + 1)] : 0.0;
+    double db = c1 < m ? R[(off + c1) * (ld + 1)] : 0.0;
+    constexpr unsigned IM = 2 * NJ - 1;
+    for (int step = 0; step < mmax; ++step) {
+      // largest remaining diagonal entry (to FP32 precision, the column in the low bits)
+      const unsigned kt = dt > 1e-18 ? (__float_as_uint((float)dt) & ~IM) | c0 : 0u;
+      const unsigned kb = db > 1e-18 ? (__float_as_uint((float)db) & ~IM) | c1 : 0u;
+      unsigned key = kt > kb ? kt : kb;
+      key = max(key, (unsigned)bm_xor32<1>((int)key));
+      key = max(key, (unsigned)bm_xor32<2>((int)key));
+      key = max(key, (unsigned)bm_xor32<4>((int)key));
+      if constexpr (JB == 4) key = max(key, (unsigned)bm_xor32<8>((int)key));
+      if (!__any(key != 0u)) break;
+      rank = step + 1;
+      const int q = (int)(key & IM);
+      if (rg == q / RPL) {
+        double vt = at[0], vb = ab[0];
+#pragma unroll
+        for (int k = 1; k < RPL; ++k) {
+          vt = (q % RPL) == k ? at[k] : vt;
+          vb = (q % RPL) == k ? ab[k] : vb;
+        }
+        row[c0] = vt;
+        row[c1] = vb;
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      const double rs = key != 0u ? bm_rsqrt(row[q]) : 0.0;
+      const double lt = row[c0] * rs, lb = row[c1] * rs;
+#pragma unroll
+      for (int k = 0; k < RPL; ++k) {
+        const double lr = row[rg * RPL + k] * rs;
+        at[k] = fma(-lr, lt, at[k]);
+        ab[k] = fma(-lr, lb, ab[k]);
+        t[k] = step == c0 ? lr : t[k];
+        b[k] = step == c1 ? lr : b[k];
+      }
+      dt = c0 == q ? 0.0 : fma(-lt, lt, dt);
+      db = c1 == q ? 0.0 : fma(-lb, lb, db);
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    }
+  }
+  // columns 0 .. rank - 1 are set: pairs over the first G0 lanes
+  int G0 = 1;
+  while (2 * G0 < rank) G0 <<= 1;
+#pragma unroll
+  for (int k = 0; k < RPL; ++k) {
+    // column j + G0 of L: in t of lane j + G0 when G0 < NJ, in b of lane j otherwise
+    double v = b[k];
+    if (G0 == 1) v = bm_xor<1>(t[k]);
+    if (G0 == 2) v = bm_xor<2>(t[k]);
+    if (G0 == 4 && NJ > 4) v = bm_xor<4>(t[k]);
+    if (G0 == 8 && NJ > 8) v = bm_xor<8>(t[k]);
+    b[k] = j < G0 ? v : 0.0;
+    t[k] = j < G0 ? t[k] : 0.0;
+  }
+  auto total = [](double x) {
+    if constexpr (JB == 3) {
+      x += bm_xor<8>(x);
+      return bm_swap_sum<16>(x);
+    } else {
+      return bm_swap_sum<32>(bm_swap_sum<16>(x));
+    }
+  };
+  for (int sweep = 0; sweep < BMAX_SWEEPS; ++sweep) {
+    bool any = false;
+    for (int G = G0; G >= 1; G >>= 1) {
+      for (int r = 1; r <= G; ++r) {
+        double pp = 0.0, qq = 0.0, pq = 0.0;
+#pragma unroll
+        for (int k = 0; k < RPL; ++k) {
+          pp = fma(t[k], t[k], pp);
+          qq = fma(b[k], b[k], qq);
+          pq = fma(t[k], b[k], pq);
+        }
+        pp = total(pp);
+        qq = total(qq);
+        pq = total(pq);
+        const bool big = pq * pq > 1.6e-29 * (pp * qq);
+        if (__any(big)) {
+          any = true;
+          // t' = c t - s b, b' = s t + c b with tan = sgn(th) / (|th| + sqrt(th^2 + 1))
+          const double th = (qq - pp) * __builtin_amdgcn_rcp(2.0 * pq);
+          const float a = fabsf((float)th);
+          const float d = a < 1e9f ? a + __builtin_amdgcn_sqrtf(fmaf(a, a, 1.0f)) : 2.0f * a;
+          const float tf = big ? copysignf(__builtin_amdgcn_rcpf(d), (float)th) : 0.0f;
+          const double tn = (double)tf;
+          const double c = bm_rsqrt(fma(tn, tn, 1.0));
+          const double s = tn * c;
+#pragma unroll
+          for (int k = 0; k < RPL; ++k) {
+            const double tk = t[k], bk = b[k];
+            t[k] = fma(-s, bk, c * tk);
+            b[k] = fma(s, tk, c * bk);
+          }
+        }
+        if (r < G) {
+          // next lane of the Gray code: the lowest set bit of r
+          if (r & 1) {
+#pragma unroll
+            for (int k = 0; k < RPL; ++k) b[k] = bm_xor<1>(b[k]);
+          } else if (r & 2) {
+#pragma unroll
+            for (int k = 0; k < RPL; ++k) b[k] = bm_xor<2>(b[k]);
+          } else if (r & 4) {
+#pragma unroll
+            for (int k = 0; k < RPL; ++k) b[k] = bm_xor<4>(b[k]);
+          } else {
+#pragma unroll
+            for (int k = 0; k < RPL; ++k) b[k] = bm_xor<8>(b[k]);
+          }
+        }
+      }
+      if (G > 1) {
+        // lanes of the lower half of a group take two t columns, the others two b
+        const int bit = G >> 1;
+        const bool up = j & bit;
+#pragma unroll
+        for (int k = 0; k < RPL; ++k) {
+          const double out = up ? t[k] : b[k];
+          const double in = bit == 1   ? bm_xor<1>(out)
+                            : bit == 2 ? bm_xor<2>(out)
+                            : bit == 4 ? bm_xor<4>(out)
+                                       : bm_xor<8>(out);
+          if (up)
+            t[k] = in;
+          else
+            b[k] = in;
+        }
+      }
+    }
+    if (!any) break;
+  }
+  double pp = 0.0, qq = 0.0;
+#pragma unroll
+  for (int k = 0; k < RPL; ++k) {
+    pp = fma(t[k], t[k], pp);
+    qq = fma(b[k], b[k], qq);
+  }
+  pp = total(pp);
+  qq = total(qq);
+  const bool ot = pp > 1e-60, ob = qq > 1e-60;
+  const int base = JB == 3 ? (lane & 32) : 0;   // row group 0 of this lane's block
+  const uint64_t low = (1ull << (1 << JB)) - 1;
+  const uint64_t mt = (__ballot(ot) >> base) & low, mb = (__ballot(ob) >> base) & low;
+  const uint64_t below = (1ull << j) - 1;
+  const int ct = off + __popcll(mt & below);
+  const int cb = off + __popcll(mt) + __popcll(mb & below);
+  const double it = bm_rsqrt(pp), ib = bm_rsqrt(qq);
+#pragma unroll
+  for (int k = 0; k < RPL; ++k) {
+    const int r = rg * RPL + k;
+    if (r < m && ot) T[(off + r) * ld + ct] = t[k] * it;
+    if (r < m && ob) T[(off + r) * ld + cb] = b[k] * ib;
+  }
+  if (rg == 0) {
+    if (ot) lam[ct] = pp;
+    if (ob) lam[cb] = qq;
+  }
 }
 
 // cyclic Jacobi on the two diagonal blocks [0, m0) and [m0, m0 + m1) of the
@@ -396,6 +647,50 @@ __device__ void bm_jacobi(BmShT<NB> &S, int m0, int m1) {
     __syncthreads();
     if (!any) break;
   }
+}
+
+// eigenvalues (S.lam) and eigenvectors (columns of S.T) of the two blocks
+// [0, m0) and [m0, m0 + m1) of S.R, columns of a block at its positions.  Blocks of
+// up to 32 go to one-sided Jacobi in the registers of one wave (both blocks, up to 16)
+// or two (S.P, free until the new projection, as scratch); larger ones (D = 3 with
+// chi > 16) to the workgroup's two-sided Jacobi in LDS.
+template <int NB>
+__device__ void bm_eigen(BmShT<NB> &S, int m0, int m1) {
+  constexpr int LD = BmShT<NB>::LD;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int mt = m0 + m1, mmax = m0 > m1 ? m0 : m1;
+  if (NB > 32 && mmax > 32) {
+    bm_jacobi<NB>(S, m0, m1);
+    for (int i = tid; i < mt; i += BT) {
+      const double l = S.R[i * LD + i];
+      S.lam[i] = l == l ? l : 0.0;   // NaN: any order, but every rank taken once
+    }
+    __syncthreads();
+    return;
+  }
+  for (int idx = tid; idx < mt * mt; idx += BT) {
+    const int i = idx / mt, j = idx - i * mt;
+    S.T[i * LD + j] = 0.0;
+  }
+  if (tid < mt) S.lam[tid] = 0.0;
+  __syncthreads();
+  // the working wave moves with the workgroup, so that workgroups that share a CU
+  // use different SIMDs
+  const int w0 = (blockIdx.x + 2 * blockIdx.y) & 3;
+  if (mmax <= 16) {
+    if (wave == w0) {
+      const bool hi = tid & 32;
+      bm_jacobi_wave<3, 4>(S.R, LD, hi ? m0 : 0, hi ? m1 : m0, mmax, S.P + (hi ? 16 : 0), S.T,
+                           S.lam);
+    }
+  } else {
+    const int blk = (wave - w0) & 3;
+    if (blk < 2)
+      // NB = 32: chi D <= 32, blocks of more than 16 only with D = 3: at most 2 chi <= 20
+      bm_jacobi_wave<4, NB == 32 ? 5 : 8>(S.R, LD, blk ? m0 : 0, blk ? m1 : m0, blk ? m1 : m0, S.P + 32 * blk,
+                           S.T, S.lam);
+  }
+  __syncthreads();
 }
 
 }  // namespace
@@ -720,14 +1015,14 @@ __global__ void __launch_bounds__(BT, NB == 32 ? 4 : 1)
           S.R[p1 * LD + p2] *= dinv;
         }
         __syncthreads();
-        bm_jacobi<NB>(S, m0, m1);
+        bm_eigen<NB>(S, m0, m1);
         // the chi leading eigenvalues (ties by position), padding excluded
         if (tid < mt && S.perm[tid] >= 0) {
-          const double lam = S.R[tid * LD + tid];
+          const double lam = S.lam[tid];
           int rank = 0;
           for (int q = 0; q < mt; ++q) {
             if (S.perm[q] < 0) continue;
-            const double lq = S.R[q * LD + q];
+            const double lq = S.lam[q];
             rank += (lq > lam) || (lq == lam && q < tid);
           }
           if (rank < kn) S.sel[rank] = tid;

@@ -500,6 +500,331 @@ __global__ void __launch_bounds__(64 * P32_W)
   }
 }
 
+// ------------------------------------------------------------ FP64 on the matrix cores
+// Amplitudes of a shared parameter vector in FP64, one wave per configuration, with
+// v_mfma_f64_16x16x4f64 and no LDS: Top and Bot of a column depend on the configuration
+// only through the local state and P_right parity of two sites each (64 combinations), so
+// a table of them is formed once per call and a configuration reads its operands from it
+// (coalesced, from L2: 2 MB at 4x4 D = 4).  Lane l, register r of a result holds
+// D[4 r + l / 16][l % 16]; an operand of k-step r holds A[l % 16][4 r + l / 16] and
+// B[4 r + l / 16][l % 16].  So a result read as the A operand is its transpose:
+//   env[a][b] (result) = A operand of  X[b][a'] = sum_a env[a][b] Top_v[a][a'],
+//   X (result)         = A operand of  env'[a'][b'] = sum_b X[b][a'] Bot_v[b][b'],
+// and the whole chain of columns stays in registers.
+// Z2: Top_v[a][a'] is nonzero only for v of one parity, given a and a'.  An even and an odd
+// v therefore share one 16 x 16 operand (pair t: Top[a][a'] of the even or odd v number t,
+// whichever a, a' allow), which halves the table and the products: two pairs at D = 4.
+// Since env[a][b] is nonzero for one parity of (a, b) only, each X entry is that of one v;
+// the sum over b mixes the two v of a pair only into entries (a', b') of the forbidden
+// parity, which are set to zero.
+// Bound by the FP64 matrix rate and L2 latency: 37 products of 64 cycles per 4x4
+// amplitude.  Measured: see peps_amp64_kernel.
+constexpr int P64_W = 4;              // configurations per workgroup
+constexpr int P64_CELL = 512;         // doubles per combination: 2 pairs x 4 k-steps x 64 lanes
+typedef double p64d4 __attribute__((ext_vector_type(4)));
+
+// number t of the even (odd = 0) or odd v below D; -1: none
+__device__ __forceinline__ int p64_v(int D, int odd, int t) {
+  const int ne = D == 1 ? 1 : D >> 1;     // even v: 0 .. ne - 1
+  const int v = odd ? ne + t : t;
+  return (odd ? v < D : t < ne) ? v : -1;
+}
+
+// Table of column operands, one workgroup per (combination, half, column):
+// tab[((y 2 + half) 64 + q) P64_CELL + ((t 2 + r / 2) 64 + lane) 2 + r % 2], q = (8 q0 + q1)
+// of the half's rows (2 state + parity each; q0 alone with one row).  First of several
+// columns (dimension 1 on the left): register 0 of pair 0, [a'][v] (k = v); last column
+// (dimension 1 on the right): pair 0, [a][v].
+__global__ void __launch_bounds__(256) peps_col_table_kernel(PepsArgs A, double *tab) {
+  const PepsGeo &g = A.g;
+  const int q = blockIdx.x, half = blockIdx.y, y = blockIdx.z, D = g.D, tid = threadIdx.x;
+  const int x0 = half ? g.tr : 0, nr = half ? g.Lx - g.tr : g.tr;
+  if (nr == 1 && q >= 8) return;
+  __shared__ double sl[2][SLICE];
+  const int q0 = nr == 2 ? q >> 3 : q, q1 = nr == 2 ? q & 7 : 0;
+  int off = 0, par = 0;
+  for (int s = 0; s < g.N; ++s) {
+    const int x = s / g.Ly, yy = s - (s / g.Ly) * g.Ly;
+    int dl, du, dd, dr;
+    site_dims(g, x, yy, dl, du, dd, dr);
+    const int n = dl * du * dd * dr;
+    if (yy == y && x >= x0 && x < x0 + nr) {
+      const int k = x - x0, pst = (k ? q1 : q0) >> 1, prs = (k ? q1 : q0) & 1;
+      par ^= pst == 1 || pst == 2;
+      for (int idx = tid; idx < n; idx += 256) {
+        const int r = idx % dr, d = (idx / dr) % dd;
+        const int e = A.dmap[off + pst * n + idx];
+        double v = e >= 0 ? A.theta[e] : 0.0;
+        if ((qpar(d, dd) * (qpar(r, dr) + prs)) & 1) v = -v;
+        sl[k][idx] = v;
+      }
+    }
+    off += 4 * n;
+  }
+  __syncthreads();
+  const int dlc = y == 0 ? 1 : D, drc = y == g.Ly - 1 ? 1 : D;
+  const int da = nr == 2 ? dlc * dlc : dlc, da2 = nr == 2 ? drc * drc : drc;
+  // the entry [a][v][a2] of Top (half 0) or Bot (half 1)
+  auto entry = [&](int a, int v, int a2) {
+    if (a >= da || a2 >= da2 || v < 0 || v >= D) return 0.0;
+    // one row: the leg v is its only vertical leg
+    if (nr == 1) return sl[0][(a * D + v) * drc + a2];
+    const int l0 = a / dlc, l1 = a % dlc, r0 = a2 / drc, r1 = a2 % drc;
+    double acc = 0.0;
+    for (int m = 0; m < D; ++m)
+      acc += half ? sl[0][((l0 * D + v) * D + m) * drc + r0] * sl[1][(l1 * D + m) * drc + r1]
+                  : sl[0][(l0 * D + m) * drc + r0] * sl[1][((l1 * D + m) * D + v) * drc + r1];
+    return acc;
+  };
+  double *cell = tab + ((int64_t)(y * 2 + half) * 64 + q) * P64_CELL;
+  for (int idx = tid; idx < P64_CELL; idx += 256) {
+    const int r = ((idx >> 7) & 1) * 2 + (idx & 1), t = idx >> 8, lane = (idx >> 1) & 63;
+    const int li = lane & 15, lk = lane >> 4, a = 4 * r + lk;
+    double v = 0.0;
+    if (y == g.Ly - 1) {
+      if (t == 0) v = entry(a, li, 0);
+    } else if (y == 0) {
+      if (t == 0 && r == 0) v = entry(0, lk, li);
+    } else {
+      // composite bond indices: the parity of both rows' legs
+      const int pa = nr == 2 ? qpar(a / D, D) ^ qpar(a % D, D) : qpar(a, D);
+      const int pb = nr == 2 ? qpar(li / D, D) ^ qpar(li % D, D) : qpar(li, D);
+      if (a < da && li < da2) v = entry(a, p64_v(D, par ^ pa ^ pb, t), li);
+    }
+    cell[idx] = v;
+  }
+}
+
+// the wave's largest exponent field of four doubles per lane
+__device__ __forceinline__ int p64_max_exp(const p64d4 &e) {
+  int m = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) m = max(m, (__double2hiint(e[r]) >> 20) & 0x7FF);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) m = max(m, __shfl_xor(m, o, 64));
+  return __builtin_amdgcn_readfirstlane(m);
+}
+
+// (sign, ln|psi|) of one configuration, site s having its down electron in bit s of dn and
+// its up electron in bit s of up; the same values in every lane
+template <int NP>
+__device__ __forceinline__ void peps_amp_wave(const PepsGeo &g, const double *__restrict__ tab,
+                                              uint32_t dn, uint32_t up, double &sign,
+                                              double &logabs) {
+  const int lane = threadIdx.x & 63, li = lane & 15, lk = lane >> 4;
+  const int Ly = g.Ly, D = g.D, br = g.Lx - g.tr;
+  const uint32_t single = dn ^ up;
+  // this lane's parity of (a, b) of the four entries of an environment
+  int fpar = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int a = 4 * r + lk;
+    const int pa = g.tr == 2 ? qpar(a / D, D) ^ qpar(a % D, D) : qpar(a, D);
+    const int pb = br == 2 ? qpar(li / D, D) ^ qpar(li % D, D) : qpar(li, D);
+    fpar |= (pa ^ pb) << r;
+  }
+  auto q8 = [&](int x, int y) {
+    const int s = x * Ly + y;
+    const uint32_t right = s + 1 < 32 ? (single >> (s + 1)) & ((1u << (Ly - 1 - y)) - 1u) : 0u;
+    return (int)((((dn >> s) & 1u) | (((up >> s) & 1u) << 1)) << 1 | (__popc(right) & 1u));
+  };
+  auto cell = [&](int y, int half) {
+    const int x0 = half ? g.tr : 0, nr = half ? br : g.tr;
+    const int q = nr == 2 ? q8(x0, y) * 8 + q8(x0 + 1, y) : q8(x0, y);
+    return reinterpret_cast<const double2 *>(tab + ((int64_t)(y * 2 + half) * 64 + q) * P64_CELL);
+  };
+  auto col_par = [&](int y) {   // singly occupied sites of column y
+    int p = 0;
+    for (int x = 0; x < g.Lx; ++x) p ^= (single >> (x * Ly + y)) & 1u;
+    return p;
+  };
+  struct Ops {
+    double2 t[NP][2], b[NP][2];
+  };
+  auto load = [&](int y, Ops &o) {
+    const double2 *ct = cell(y, 0), *cb = cell(y, 1);
+#pragma unroll
+    for (int t = 0; t < NP; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        o.t[t][h] = ct[(t * 2 + h) * 64 + lane];
+        o.b[t][h] = cb[(t * 2 + h) * 64 + lane];
+      }
+  };
+  p64d4 env = {lane == 0 ? 1.0 : 0.0, 0.0, 0.0, 0.0};
+  int esc = 0, par = 0;
+  Ops cur, nxt;
+  int y = 0;
+  if (Ly > 1) {
+    const double ft = cell(0, 0)[lane].x, fb = cell(0, 1)[lane].x;
+    load(1, cur);
+    const p64d4 z = {0.0, 0.0, 0.0, 0.0};
+    env = __builtin_amdgcn_mfma_f64_16x16x4f64(ft, fb, z, 0, 0, 0);
+    par = col_par(0);
+    y = 1;
+  } else {
+    load(0, cur);
+  }
+  for (; y < Ly - 1; ++y) {
+    load(y + 1, nxt);
+    p64d4 out[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+    p64d4 X[NP];
+#pragma unroll
+    for (int t = 0; t < NP; ++t) X[t] = (p64d4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < NP; ++t)
+        X[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+            env[r], r & 1 ? cur.t[t][r >> 1].y : cur.t[t][r >> 1].x, X[t], 0, 0, 0);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int t = 0; t < NP; ++t)
+        out[NP == 2 ? t : r & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+            X[t][r], r & 1 ? cur.b[t][r >> 1].y : cur.b[t][r >> 1].x, out[NP == 2 ? t : r & 1], 0,
+            0, 0);
+    par ^= col_par(y);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      env[r] = ((fpar >> r) & 1) == par ? out[0][r] + out[1][r] : 0.0;
+    // scaled by a power of two (no rounding), the exponent carried aside; all zero, infinite
+    // or NaN: left alone
+    const int ex = p64_max_exp(env);
+    if (ex > 0 && ex < 0x7FF) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) env[r] = ldexp(env[r], 1023 - ex);
+      esc += ex - 1023;
+    }
+    cur = nxt;
+  }
+  // last column: X[b][v] = sum_a env[a][b] Top[a][v], psi = sum X Bot
+  p64d4 X = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    X = __builtin_amdgcn_mfma_f64_16x16x4f64(env[r], r & 1 ? cur.t[0][r >> 1].y : cur.t[0][r >> 1].x,
+                                             X, 0, 0, 0);
+  double v = 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) v = fma(X[r], r & 1 ? cur.b[0][r >> 1].y : cur.b[0][r >> 1].x, v);
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  const int P = __popc(single);
+  if ((P * (P - 1) / 2) & 1) v = -v;
+  const double lo = log(1e-45);
+  if (v == 0.0 || !std::isfinite(v)) {
+    sign = 0.0;
+    logabs = lo;
+  } else {
+    sign = v > 0.0 ? 1.0 : -1.0;
+    logabs = fmax(log(fabs(v)) + esc * 0.693147180559945309417, lo);
+  }
+}
+
+// Measured, 4x4 D = 4: 53 k configurations in 126 us (2.5 ms with one workgroup per
+// configuration and the columns formed in LDS).
+template <int NP>
+__global__ void __launch_bounds__(64 * P64_W)
+    peps_amp64_kernel(PepsGeo g, const double *__restrict__ tab, int64_t rows,
+                      const int64_t *__restrict__ cfg, const int32_t *__restrict__ flag,
+                      double *sign, double *logabs) {
+  const int lane = threadIdx.x & 63;
+  const int64_t w = (int64_t)blockIdx.x * P64_W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w >= rows) return;
+  if (flag && !(flag[w] & 1)) return;
+  const int c = lane < g.N ? (int)cfg[w * g.N + lane] : 0;
+  const uint32_t dn = (uint32_t)__ballot(c & 1), up = (uint32_t)__ballot(c & 2);
+  double s, l;
+  peps_amp_wave<NP>(g, tab, dn, up, s, l);
+  if (lane == 0) {
+    sign[w] = s;
+    logabs[w] = l;
+  }
+}
+
+// A run of a sweep's edges for every walker, one wave per walker: proposal, amplitude and
+// Metropolis test per edge with the configuration in two bit masks (the same draws, order
+// and test as nnbf_propose_kernel / peps_accept_kernel).  One launch instead of four per
+// edge, and no proposal configurations in memory.
+struct PepsEdges {
+  enum { MAX = 128 };
+  int n, first;             // edges of this launch, and the number of the first in the sweep
+  uint8_t i[MAX], j[MAX];
+};
+
+// Measured, 4x4 D = 4, 2048 walkers, 24 edges: 145 us (2.8 ms in 96 launches).
+template <int NP>
+__global__ void __launch_bounds__(64 * P64_W)
+    peps_sweep64_kernel(PepsGeo g, const double *__restrict__ tab, int64_t B, PepsEdges ed,
+                        int64_t sweep, uint64_t seed, double keep_rate,
+                        const double *__restrict__ u_choice, const uint8_t *__restrict__ bits,
+                        const double *__restrict__ u_acc, int64_t *cfg, double *sign,
+                        double *logabs, int64_t *n_accept) {
+  const int lane = threadIdx.x & 63;
+  const int64_t w = (int64_t)blockIdx.x * P64_W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (w >= B) return;
+  const int c = lane < g.N ? (int)cfg[w * g.N + lane] : 0;
+  uint32_t dn = (uint32_t)__ballot(c & 1), up = (uint32_t)__ballot(c & 2);
+  double sg = sign[w], la = logabs[w];
+  int n_acc = 0;
+  for (int e = 0; e < ed.n; ++e) {
+    const int i = ed.i[e], j = ed.j[e];
+    const int si = ((dn >> i) & 1) | (((up >> i) & 1) << 1);
+    const int sj = ((dn >> j) & 1) | (((up >> j) & 1) << 1);
+    if (si == sj) continue;
+    double uc, ua;
+    int b0, b2;
+    if (u_choice == nullptr) {
+      const u32x4 o = philox4x32_10((uint32_t)(ed.first + e), (uint32_t)sweep, (uint32_t)w, 0u,
+                                    (uint32_t)seed, (uint32_t)(seed >> 32));
+      uc = u53(o.x, o.y);
+      ua = u53(o.z, o.w);
+      b0 = o.y & 1u;
+      b2 = (o.y >> 1) & 1u;
+    } else {
+      const int64_t k = (int64_t)e * B + w;
+      uc = u_choice[k];
+      ua = u_acc[k];
+      b0 = bits[k] & 1;
+      b2 = (bits[k] >> 1) & 1;
+    }
+    const int nmi = si == 0 ? 0 : (si == 3 ? 2 : 1), nmj = sj == 0 ? 0 : (sj == 3 ? 2 : 1);
+    const int dnum = nmi > nmj ? nmi - nmj : nmj - nmi;
+    int ni, nj;
+    if (uc < keep_rate || dnum == 1) {
+      ni = sj;
+      nj = si;
+    } else if (dnum == 0) {
+      ni = b0 ? 3 : 0;
+      nj = b0 ? 0 : 3;
+    } else {
+      ni = b2 ? 2 : 1;
+      nj = b2 ? 1 : 2;
+    }
+    const uint32_t keep = ~((1u << i) | (1u << j));
+    const uint32_t dn2 = (dn & keep) | ((uint32_t)(ni & 1) << i) | ((uint32_t)(nj & 1) << j);
+    const uint32_t up2 = (up & keep) | ((uint32_t)(ni >> 1) << i) | ((uint32_t)(nj >> 1) << j);
+    double ps, pl;
+    peps_amp_wave<NP>(g, tab, __builtin_amdgcn_readfirstlane(dn2),
+                      __builtin_amdgcn_readfirstlane(up2), ps, pl);
+    const double ratio = exp(2.0 * (pl - la));
+    // every lane holds the same values: one decision for the wave
+    if (__builtin_amdgcn_readfirstlane(ua < ratio ? 1 : 0)) {
+      dn = dn2;
+      up = up2;
+      sg = ps;
+      la = pl;
+      ++n_acc;
+    }
+  }
+  if (lane < g.N) cfg[w * g.N + lane] = ((dn >> lane) & 1) | (((up >> lane) & 1) << 1);
+  if (lane == 0) {
+    sign[w] = sg;
+    logabs[w] = la;
+    if (n_accept) n_accept[w] += n_acc;
+  }
+}
+
 // ------------------------------------------------------------ environment reuse
 // Per-walker cache of the column environments of the exact contraction:
 // L_y = columns 0 .. y-1 absorbed from the left, R_y = columns y .. Ly-1
@@ -1138,6 +1463,8 @@ struct PepsWs {
   double *coeffs, *csign, *clog;
   // FP32 amplitudes of a shared parameter vector: the signed slice table
   float *tbl;
+  // FP64 amplitudes of a shared parameter vector: the column operands
+  double *ctab;
   // chi-truncated boundary MPS: slots of bm_pass configurations (bm_gpass
   // for the log-derivative's per-row environments); the sweep's boundary
   // cache of the B walkers (plain fPEPS)
@@ -1165,6 +1492,11 @@ bool use_bmps(const vmcx_peps_model &m) {
   int64_t big = 1;
   for (int i = 0; i < m.Lx - m.Lx / 2; ++i) big *= m.D;
   return m.chi < big;
+}
+
+// exact FP64 amplitudes of one parameter vector (plain fPEPS): from the column table
+bool table64(const vmcx_peps_model &m) {
+  return m.hidden <= 0 && !m.amp_fp32 && !use_bmps(m);
 }
 
 PepsWs peps_layout(const vmcx_peps_model &m, int64_t B, int64_t chunk, int n_edges,
@@ -1204,6 +1536,7 @@ PepsWs peps_layout(const vmcx_peps_model &m, int64_t B, int64_t chunk, int n_edg
   L.csign = (double *)take((size_t)T * 8);
   L.clog = (double *)take((size_t)T * 8);
   L.tbl = (float *)take(m.amp_fp32 && H == 0 ? (size_t)N * 8 * 256 * 4 : 0);
+  L.ctab = (double *)take(table64(m) ? (size_t)m.Ly * 2 * 64 * P64_CELL * 8 : 0);
   if (use_bmps(m)) {
     L.bm_pass = rows < BM_PASS ? (rows > 0 ? rows : 1) : BM_PASS;
     L.bm_gpass = chunk < BM_GPASS ? (chunk > 0 ? chunk : 1) : BM_GPASS;
@@ -1306,7 +1639,16 @@ int mlp_theta(const vmcx_peps_model &m, const PepsWs &L, int64_t rows, const int
   return 0;
 }
 
-// amplitudes of `rows` configurations (rows <= chunk for NN-fTNS)
+// what amp_rows and the sweep read besides the parameters: formed once per entry point
+int amp_tables(const vmcx_peps_model &m, const PepsWs &L, hipStream_t st) {
+  if (!table64(m)) return 0;
+  hipLaunchKernelGGL(peps_col_table_kernel, dim3(64, 2, (unsigned)m.Ly), dim3(256), 0, st,
+                     args_of(m, m.theta, 0), L.ctab);
+  VMCX_LAUNCHED();
+  return 0;
+}
+
+// amplitudes of `rows` configurations (rows <= chunk for NN-fTNS); amp_tables first
 int amp_rows(const vmcx_peps_model &m, const PepsWs &L, int64_t rows, const int64_t *cfg,
              const int32_t *flag, double *sign, double *logabs, hipStream_t st) {
   if (rows == 0) return 0;
@@ -1319,7 +1661,15 @@ int amp_rows(const vmcx_peps_model &m, const PepsWs &L, int64_t rows, const int6
   if (use_bmps(m))
     return bmps_amplitudes(m.Lx, m.Ly, m.D, m.chi, A.dmap, A.theta, A.theta_stride, rows, cfg,
                            flag, sign, logabs, L.bm, L.bm_pass, st);
-  if (m.amp_fp32) {
+  if (table64(m)) {
+    const dim3 grid((unsigned)((rows + P64_W - 1) / P64_W)), blk(64 * P64_W);
+    if (m.D > 2)
+      hipLaunchKernelGGL(peps_amp64_kernel<2>, grid, blk, 0, st, A.g, L.ctab, rows, cfg, flag,
+                         sign, logabs);
+    else
+      hipLaunchKernelGGL(peps_amp64_kernel<1>, grid, blk, 0, st, A.g, L.ctab, rows, cfg, flag,
+                         sign, logabs);
+  } else if (m.amp_fp32) {
     const float *tbl = nullptr;
     if (m.hidden == 0) {
       const int64_t ne = (int64_t)A.g.N * 8 * 256;
@@ -1402,6 +1752,10 @@ int peps_forward(const vmcx_peps_model *m, int64_t B, const int64_t *cfg, void *
   const PepsWs L = peps_layout(*m, B, chunk, 0, (char *)ws);
   VMCX_CHECK_ARG((int64_t)L.bytes <= ws_bytes, "workspace too small");
   const int N = m->Lx * m->Ly;
+  {
+    const int rc = amp_tables(*m, L, st);
+    if (rc) return rc;
+  }
   for (int64_t r0 = 0; r0 < B; r0 += chunk) {
     const int64_t rows = (B - r0 < chunk) ? B - r0 : chunk;
     const int rc = amp_rows(*m, L, rows, cfg + r0 * N, nullptr, sign + r0, logabs + r0, st);
@@ -1428,6 +1782,30 @@ int peps_sweep(const vmcx_peps_model *m, int64_t B, int n_edges, const int32_t *
   for (int e = 0; e < n_edges; ++e) {
     const int i = edges_host[2 * e], j = edges_host[2 * e + 1];
     VMCX_CHECK_ARG(i >= 0 && i < N && j >= 0 && j < N && i != j, "edge out of range");
+  }
+  if (table64(*m)) {
+    int rc = amp_tables(*m, L, st);
+    if (rc) return rc;
+    const PepsGeo g = args_of(*m, m->theta, 0).g;
+    const dim3 grid((unsigned)((B + P64_W - 1) / P64_W)), blk(64 * P64_W);
+    for (int sw = 0; sw < n_sweeps; ++sw)
+      for (int e0 = 0; e0 < n_edges; e0 += PepsEdges::MAX) {
+        PepsEdges ed{};
+        ed.n = n_edges - e0 < PepsEdges::MAX ? n_edges - e0 : (int)PepsEdges::MAX;
+        ed.first = e0;
+        for (int e = 0; e < ed.n; ++e) {
+          ed.i[e] = (uint8_t)edges_host[2 * (e0 + e)];
+          ed.j[e] = (uint8_t)edges_host[2 * (e0 + e) + 1];
+        }
+        const size_t di = ((size_t)sw * n_edges + e0) * B;
+        const auto kern = m->D > 2 ? peps_sweep64_kernel<2> : peps_sweep64_kernel<1>;
+        hipLaunchKernelGGL(kern, grid, blk, 0, st, g, L.ctab, B, ed, sweep_offset + sw, seed,
+                           1.0 - hopping_rate, u_choice ? u_choice + di : nullptr,
+                           bits ? bits + di : nullptr, u_acc ? u_acc + di : nullptr, cfg, sign,
+                           logabs, n_accept);
+        VMCX_LAUNCHED();
+      }
+    return 0;
   }
   const unsigned gw = (unsigned)((B + 255) / 256);
   const unsigned gc = (unsigned)((B * N + 255) / 256);
@@ -1506,6 +1884,8 @@ int peps_local_energy(const vmcx_peps_model *m, int64_t B, int n_edges, const in
                               L.cparent, L.cmove, L.bmc, L.csign, L.clog, st);
     if (rc) return rc;
   } else {
+    const int rt = amp_tables(*m, L, st);
+    if (rt) return rt;
     for (int64_t r0 = 0; r0 < T; r0 += chunk) {
       const int64_t rows = (T - r0 < chunk) ? T - r0 : chunk;
       const int rc = amp_rows(*m, L, rows, L.etas + r0 * N, nullptr, L.csign + r0, L.clog + r0,

@@ -93,6 +93,23 @@ int vmcx_slater_sweep(int64_t B, int n_sites, int n_f, const double *M,
                       double *sign, double *logabs, int32_t *since_refresh,
                       int64_t *n_accept, const int64_t *sweep_offset_dev, void *stream);
 
+/* since_refresh of a walker whose state predates the present parameters. */
+#define VMCX_SLATER_STALE (1 << 30)
+/* Compares n parameters (FP64, or FP32 with f32 = 1) bit by bit with `snapshot`, on the
+ * device: when they differ, or force = 1, copies them to `snapshot`, widens FP32 ones to
+ * `wide` (may be NULL) and sets the B entries of since_refresh to VMCX_SLATER_STALE.  A
+ * vmcx_slater_refresh with only_if_since = VMCX_SLATER_STALE then rebuilds the walkers
+ * whose parameters changed and no others.  No counterpart in the reference. */
+int vmcx_slater_mark_params(int64_t n, const void *params, int f32, void *snapshot, double *wide,
+                            int force, int64_t B, int32_t *since_refresh, void *stream);
+
+/* counts[0] <- samples with a non-finite sign or ln|psi|, counts[1] <- rows of O ([B][n],
+ * row stride ld; o_dtype 0 = FP64, 1 = FP32) whose sum is not finite (counts: 2 int64 on the
+ * device).  Replaces: _check_grads_amps (GPU/vmc_utils.py:1330-1386). */
+int vmcx_count_nonfinite(int64_t B, int64_t n, const void *O, int o_dtype, int64_t ld,
+                         const double *sign, const double *logabs, int64_t *counts,
+                         void *stream);
+
 /* counter[0] += inc on `stream` (a one-thread kernel: graph-capturable, no
  * memset node).  Advances the device draw counters of vmcx_slater_sweep and
  * vmcx_lp_propose_given / vmcx_lp_accept inside a captured graph.  No

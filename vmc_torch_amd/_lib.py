@@ -64,6 +64,8 @@ _SIGNATURES = {
     "vmcx_nnbf_workspace_bytes": (_I64, [_P, _I64, _I64, _I]),
     "vmcx_nnbf_forward": (_I, [_P, _I64, _P, _P, _I64, _I64, _P, _P, _P, _P]),
     "vmcx_nnbf_forward_moved": (_I, [_P, _I64, _P, _P, _P, _P, _I64, _I64, _P, _P, _P, _P]),
+    "vmcx_slater_mark_params": (_I, [_I64, _P, _I, _P, _P, _I, _I64, _P, _P]),
+    "vmcx_count_nonfinite": (_I, [_I64, _I64, _P, _I, _I64, _P, _P, _P, _P]),
     "vmcx_masked_rows": (_I, [_I64, _I64, _P, _P, _P, _P]),
     "vmcx_nnbf_sweep": (_I, [_P, _I64, _I, _P, _D, _I, _U64, _I64, _P, _P, _P, _P, _P,
                              _P, _P, _P, _P, _I64, _P]),

@@ -378,6 +378,17 @@ int vmcx_lp_accept(int64_t B, int n_sites, uint64_t seed, int64_t step, const do
                                    accepted, (hipStream_t)stream, step_dev));
 }
 
+int vmcx_slater_mark_params(int64_t n, const void *params, int f32, void *snapshot, double *wide,
+                            int force, int64_t B, int32_t *since_refresh, void *stream) {
+  return status_of(vmcx::slater_mark_params(n, params, f32, snapshot, wide, force, B,
+                                            since_refresh, (hipStream_t)stream));
+}
+int vmcx_count_nonfinite(int64_t B, int64_t n, const void *O, int o_dtype, int64_t ld,
+                         const double *sign, const double *logabs, int64_t *counts,
+                         void *stream) {
+  return status_of(vmcx::count_nonfinite(B, n, O, o_dtype, ld, sign, logabs, counts,
+                                         (hipStream_t)stream));
+}
 int vmcx_counter_add(int64_t *counter, int64_t inc, void *stream) {
   return status_of(vmcx::counter_add(counter, inc, (hipStream_t)stream));
 }

@@ -231,6 +231,10 @@ int lp_accept(int64_t B, int N, uint64_t seed, int64_t step, const double *u_acc
               const double *plog, const double *logq_f, const double *logq_r, int64_t *cfg,
               double *sign, double *logabs, int64_t *n_accept, uint8_t *accepted,
               hipStream_t st, const int64_t *step_dev = nullptr);
+int slater_mark_params(int64_t n, const void *params, int f32, void *snapshot, double *wide,
+                       int force, int64_t B, int32_t *since, hipStream_t st);
+int count_nonfinite(int64_t B, int64_t n, const void *O, int o_dtype, int64_t ld,
+                    const double *sign, const double *logabs, int64_t *counts, hipStream_t st);
 int counter_add(int64_t *ctr, int64_t inc, hipStream_t st);
 int64_t lp_backward_workspace_bytes(int C, int64_t B);
 int lp_backward(const float *P, int C, int Lx, int Ly, int64_t B, const int64_t *cfg,

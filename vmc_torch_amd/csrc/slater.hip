@@ -12,6 +12,9 @@
 //     per lane;
 //   * the log-derivative row of an occupied orbital is a contiguous column
 //     of A^-1 in HBM (column k stored at ainv + (b*NFP + k)*NFP).
+#include <cmath>
+
+#include "../../include/vmcx.h"
 #include "gj.h"
 #include "kernels.h"
 
@@ -745,6 +748,103 @@ __global__ void counter_add_kernel(int64_t *ctr, int64_t inc) { ctr[0] += inc; }
 int counter_add(int64_t *ctr, int64_t inc, hipStream_t st) {
   VMCX_CHECK_ARG(ctr != nullptr, "null counter");
   hipLaunchKernelGGL(counter_add_kernel, dim3(1), dim3(1), 0, st, ctr, inc);
+  VMCX_LAUNCHED();
+  return 0;
+}
+
+// Parameters against the copy that the walker state was built from, without a host
+// synchronisation: when a byte differs (or force), the copy and the FP64 widening of FP32
+// parameters are brought up to date and every walker's since_refresh becomes STALE, so that
+// a refresh with only_if_since = STALE rebuilds the walkers if, and only if, the
+// parameters changed.  One workgroup: M is at most 64 KB, a few us; the value comparison
+// it replaces (concatenation, equality, reduction, host read) held the device idle for
+// some 40 us.
+__global__ void __launch_bounds__(1024)
+    mark_params_kernel(int64_t words, const uint32_t *__restrict__ params, uint32_t *snapshot,
+                       double *wide, int force, int64_t B, int32_t *since, int32_t stale) {
+  __shared__ int any;
+  if (threadIdx.x == 0) any = force;
+  __syncthreads();
+  bool diff = false;
+  for (int64_t i = threadIdx.x; i < words; i += 1024) diff |= params[i] != snapshot[i];
+  if (diff) any = 1;
+  __syncthreads();
+  if (!any) return;
+  for (int64_t i = threadIdx.x; i < words; i += 1024) {
+    const uint32_t v = params[i];
+    snapshot[i] = v;
+    if (wide) wide[i] = (double)__uint_as_float(v);
+  }
+  for (int64_t w = threadIdx.x; w < B; w += 1024) since[w] = stale;
+}
+
+int slater_mark_params(int64_t n, const void *params, int f32, void *snapshot, double *wide,
+                       int force, int64_t B, int32_t *since, hipStream_t st) {
+  VMCX_CHECK_ARG(n >= 0 && B >= 0, "negative size");
+  VMCX_CHECK_ARG(n == 0 || (params && snapshot), "null pointer");
+  VMCX_CHECK_ARG(B == 0 || since, "null pointer");
+  VMCX_CHECK_ARG(f32 || !wide, "wide is for FP32 parameters");
+  hipLaunchKernelGGL(mark_params_kernel, dim3(1), dim3(1024), 0, st, f32 ? n : 2 * n,
+                     (const uint32_t *)params, (uint32_t *)snapshot, wide, force, B, since,
+                     (int32_t)VMCX_SLATER_STALE);
+  VMCX_LAUNCHED();
+  return 0;
+}
+
+// counts[0]: samples whose sign or ln|psi| is not finite; counts[1]: rows of O whose sum is
+// not (a NaN or Inf anywhere in a row).  One wave per row, one read of O, 16 bytes a lane
+// where the rows are aligned to that.
+__global__ void count_zero_kernel(int64_t *counts) { counts[threadIdx.x] = 0; }
+
+template <typename T>
+__global__ void __launch_bounds__(256)
+    count_nonfinite_kernel(int64_t B, int64_t n, const T *__restrict__ O, int64_t ld, int vec,
+                           const double *__restrict__ sign, const double *__restrict__ logabs,
+                           int64_t *counts) {
+  constexpr int V = 16 / sizeof(T);
+  const int lane = threadIdx.x & 63;
+  const int64_t w = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (w >= B) return;
+  const T *row = O + w * ld;
+  T s = 0;
+  int64_t i = 0;
+  if (vec) {
+    const int64_t nv = n / V;
+    for (int64_t q = lane; q < nv; q += 64) {
+      T v[V];
+      *reinterpret_cast<int4 *>(v) = reinterpret_cast<const int4 *>(row)[q];
+#pragma unroll
+      for (int k = 0; k < V; ++k) s += v[k];
+    }
+    i = nv * V;
+  }
+  for (int64_t q = i + lane; q < n; q += 64) s += row[q];
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+  if (lane == 0) {
+    if (!std::isfinite(sign[w]) || !std::isfinite(logabs[w]))
+      atomicAdd((unsigned long long *)&counts[0], 1ull);
+    if (!std::isfinite(s)) atomicAdd((unsigned long long *)&counts[1], 1ull);
+  }
+}
+
+int count_nonfinite(int64_t B, int64_t n, const void *O, int o_dtype, int64_t ld,
+                    const double *sign, const double *logabs, int64_t *counts, hipStream_t st) {
+  VMCX_CHECK_ARG(B >= 0 && n >= 0 && ld >= n, "bad sizes");
+  VMCX_CHECK_ARG(o_dtype == 0 || o_dtype == 1, "o_dtype must be 0 (f64) or 1 (f32)");
+  VMCX_CHECK_ARG(counts && (B == 0 || (sign && logabs && (n == 0 || O))), "null pointer");
+  VMCX_CHECK_ARG(B <= 0x7fffffff, "B too large for one grid");
+  hipLaunchKernelGGL(count_zero_kernel, dim3(1), dim3(2), 0, st, counts);
+  if (B > 0) {
+    const dim3 grid((unsigned)((B + 3) / 4)), blk(256);
+    const int64_t esz = o_dtype == 0 ? 8 : 4;
+    const int vec = ((uintptr_t)O & 15) == 0 && (ld * esz) % 16 == 0;
+    if (o_dtype == 0)
+      hipLaunchKernelGGL(count_nonfinite_kernel<double>, grid, blk, 0, st, B, n,
+                         (const double *)O, ld, vec, sign, logabs, counts);
+    else
+      hipLaunchKernelGGL(count_nonfinite_kernel<float>, grid, blk, 0, st, B, n,
+                         (const float *)O, ld, vec, sign, logabs, counts);
+  }
   VMCX_LAUNCHED();
   return 0;
 }

@@ -122,6 +122,39 @@ def slater_sweep(M, edges, configs, state, n_sweeps=1, seed=0, sweep_offset=0,
              ptr(state.n_accept), ptr(offset_dev), stream_ptr(M.device)))
 
 
+SLATER_STALE = 1 << 30     # VMCX_SLATER_STALE
+
+
+def slater_mark_params(M, snapshot, wide=None, state=None, force=False):
+    """Mark the walkers of `state` stale if M differs from `snapshot` (same
+    dtype and size) or force; snapshot and `wide` (FP64 copy of FP32 M) are
+    then brought up to date.  Nothing is read back to the host."""
+    f32 = M.dtype == torch.float32
+    require(M, torch.float32 if f32 else F64, "M")
+    require(snapshot, M.dtype, "snapshot", (M.numel(),), M.device)
+    if f32:
+        require(wide, F64, "wide", tuple(M.shape), M.device)
+    since = None if state is None else state.since_refresh
+    B = 0 if since is None else since.shape[0]
+    check(lib().vmcx_slater_mark_params(M.numel(), ptr(M), 1 if f32 else 0, ptr(snapshot),
+                                        ptr(wide) if f32 else None, 1 if force else 0, B,
+                                        ptr(since), stream_ptr(M.device)))
+
+
+def count_nonfinite(O, sign, logabs):
+    """[samples with a non-finite sign or ln|psi|, rows of O with a
+    non-finite sum] as an int64 device tensor."""
+    if O.dtype not in (torch.float64, torch.float32):
+        raise TypeError("O must be float64 or float32")
+    B, n = O.shape
+    require(sign, F64, "sign", (B,), O.device)
+    require(logabs, F64, "logabs", (B,), O.device)
+    counts = torch.empty(2, dtype=I64, device=O.device)
+    check(lib().vmcx_count_nonfinite(B, n, ptr(O), 0 if O.dtype == F64 else 1, O.stride(0),
+                                     ptr(sign), ptr(logabs), ptr(counts), stream_ptr(O.device)))
+    return counts
+
+
 def counter_add(counter, inc):
     """counter[0] += inc on the current stream (graph-capturable)."""
     require(counter, I64, "counter", (1,))

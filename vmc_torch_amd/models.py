@@ -119,6 +119,7 @@ class SlaterDeterminant_GPU(WavefunctionModel_GPU):
         self.n_orbitals = n_orbitals
         self.n_fermions = n_fermions
         self.n_sites = n_orbitals // 2
+        self._built_from = None     # the M that the walker state was built from
         self._m64 = None
 
     @property
@@ -132,39 +133,59 @@ class SlaterDeterminant_GPU(WavefunctionModel_GPU):
     graph_safe = True
 
     def _prepare_device_data(self):
-        if self.params_changed():
-            self._state_key = None      # the walker state predates the change
-        self._m_f64()
+        self._mark(self._state)
+
+    def _mark(self, state, force=False):
+        """Mark `state`'s walkers stale if M changed since it was built (force:
+        in any case), comparing on the device, and bring the FP64 copy of an
+        FP32 M up to date."""
+        M = self.M.detach()
+        if self._built_from is None or self._built_from.device != M.device or \
+                self._built_from.dtype != M.dtype:
+            self._built_from = torch.empty(M.numel(), dtype=M.dtype, device=M.device)
+            self._m64 = torch.empty(M.shape, dtype=torch.float64, device=M.device) \
+                if self.fp32 else None
+            force = True
+        kernels.slater_mark_params(M, self._built_from, self._m64, state, force)
 
     def _m_f64(self):
-        """M in FP64 for the exact refresh (M itself in the plain form)."""
+        """M in FP64 for the exact refresh (M itself in the plain form; the
+        copy that _mark keeps otherwise)."""
         M = self.M.detach()
         if not self.fp32:
             return M
-        if self._m64 is None or self._m64[0] is not self._snapshot:
-            self._m64 = (self._snapshot, M.to(torch.float64).contiguous())
-        return self._m64[1]
+        if self._m64 is None or self._m64.device != M.device:
+            self._mark(self._state)
+        return self._m64
 
     def forward_log(self, x):
-        self.params_changed()
-        return kernels.slater_refresh(self._m_f64(), x.contiguous())
+        M = self.M.detach()
+        return kernels.slater_refresh(M.to(torch.float64).contiguous() if self.fp32 else M,
+                                      x.contiguous())
 
     def walker_state(self, fxs, refresh=False):
         """State for the walker batch `fxs`, rebuilt exactly when fxs or M
-        changed since it was last built."""
-        changed = self.params_changed()
-        if not refresh and not changed and self._state is not None and \
-                self._state_key == self._walker_key(fxs):
-            return self._state
+        changed since it was last built (M: decided on the device, so nothing
+        waits for the host)."""
         B = fxs.shape[0]
-        st = self._state
+        st, key = self._state, self._walker_key(fxs)
         if st is None or st.ainv.shape[0] != B or st.ainv.device != fxs.device or \
                 st.ainv.dtype != self.M.dtype:
-            st = kernels.SlaterWalkerState.empty(B, self.n_sites, self.n_fermions, fxs.device,
-                                                 dtype=self.M.dtype)
-        kernels.slater_refresh(self._m_f64(), fxs, st)
-        self._state, self._state_key = st, self._walker_key(fxs)
+            st, refresh = kernels.SlaterWalkerState.empty(
+                B, self.n_sites, self.n_fermions, fxs.device, dtype=self.M.dtype), True
+        if refresh or self._state_key != key:
+            self._mark(st, force=True)
+            kernels.slater_refresh(self._m_f64(), fxs, st)
+            self._state, self._state_key = st, key
+        else:
+            if not getattr(self, "_frozen", False):
+                self._mark(st)
+            kernels.slater_refresh(self._m_f64(), fxs, st, only_if_since=kernels.SLATER_STALE)
         return st
+
+    def accept_counts(self, fxs):
+        """Accepted moves per walker so far ([B] int64, counted on in place)."""
+        return self.walker_state(fxs).n_accept
 
     def mcmc_sweep(self, fxs, edges, n_sweeps, seed, sweep_offset, hopping_rate=0.25,
                    refresh_every=64, draws=None):
@@ -392,6 +413,10 @@ class NNBF_GPU(WavefunctionModel_GPU):
         self._state, self._state_key = st, self._walker_key(fxs)
         return st
 
+    def accept_counts(self, fxs):
+        """Accepted moves per walker so far ([B] int64, counted on in place)."""
+        return self.walker_state(fxs)["n_accept"]
+
     def mcmc_sweep(self, fxs, edges, n_sweeps, seed, sweep_offset, hopping_rate=0.25,
                    refresh_every=64, draws=None):
         st = self.walker_state(fxs)
@@ -557,6 +582,7 @@ class fPEPS_Model_GPU(WavefunctionModel_GPU):
         # walker's cached boundaries (same amplitudes, bit for bit)
         self.bmps_cache = True
         self._struct_obj = None
+        self._struct_at = None
         self._ws = {}
 
     # ------------------------------------------------------ device struct
@@ -564,19 +590,31 @@ class fPEPS_Model_GPU(WavefunctionModel_GPU):
         return None
 
     def _sync(self):
-        changed = self.params_changed()
-        if changed or self._struct_obj is None:
-            for p in self.params:
-                if not p.data.is_contiguous():
-                    p.data = p.data.contiguous()
+        """The struct the kernels read: it points to the parameters
+        themselves, so only a moved tensor needs a new one."""
+        for p in self.params:
+            if not p.data.is_contiguous():
+                p.data = p.data.contiguous()
+        at = tuple(p.data_ptr() for p in self.params) + (self.dense_map.data_ptr(),)
+        if self._struct_obj is None or self._struct_at != at:
             self._struct_obj = kernels.peps_struct(
                 self.Lx, self.Ly, self.D, self.dense_map, self.params[0].data,
                 self._nn_dict(), 0 if self.act_name == "relu" else 1, self.eta, self.mode,
                 amp_fp32=self.amp == "fp32", chi=self.chi if self._bmps else 0,
                 bmps_cache=self.bmps_cache)
+            self._struct_at = at
             self._state_key = None
-            return True
-        return False
+
+    # True where a walker's amplitude is cheaper to form again than the
+    # parameters are to compare on the host (plain fPEPS, exact contraction)
+    @property
+    def _cheap_state(self):
+        return not self._bmps and getattr(self, "hidden", 0) == 0
+
+    def _prepare_device_data(self):
+        self._sync()
+        if self._cheap_state or self.params_changed():
+            self._state_key = None
 
     def _ws_for(self, B, chunk, n_edges, device):
         return kernels.peps_workspace(self._struct_obj, B, chunk, n_edges, device, self._ws)
@@ -644,8 +682,11 @@ class fPEPS_Model_GPU(WavefunctionModel_GPU):
 
     # --------------------------------------------------------- walker state
     def walker_state(self, fxs, refresh=False):
-        changed = self._sync()
-        if not refresh and not changed and self._state is not None and \
+        self._sync()
+        frozen = getattr(self, "_frozen", False)
+        if not frozen and not self._cheap_state and self.params_changed():
+            self._state_key = None
+        if not refresh and (frozen or not self._cheap_state) and self._state is not None and \
                 self._state_key == self._walker_key(fxs):
             return self._state
         B = fxs.shape[0]
@@ -656,6 +697,10 @@ class fPEPS_Model_GPU(WavefunctionModel_GPU):
                            else torch.zeros(B, dtype=torch.int64, device=fxs.device))}
         self._state, self._state_key = st, self._walker_key(fxs)
         return st
+
+    def accept_counts(self, fxs):
+        """Accepted moves per walker so far ([B] int64, counted on in place)."""
+        return self.walker_state(fxs)["n_accept"]
 
     def mcmc_sweep(self, fxs, edges, n_sweeps, seed, sweep_offset, hopping_rate=0.25,
                    refresh_every=64, draws=None):
@@ -778,6 +823,10 @@ class fPEPS_Model_reuse_GPU(fPEPS_Model_GPU):
         super().__init__(Lx, Ly, D, theta=theta, generator=generator, dtype=dtype,
                          max_bond=max_bond, chunk=chunk)
         self.radius = 0
+
+    @property
+    def _cheap_state(self):
+        return False      # the sweep's amplitudes are the reuse path's own
 
     def _ws_reuse(self, B, chunk, n_edges, device):
         return kernels.peps_workspace(self._struct_obj, B, chunk, n_edges, device, self._ws,

@@ -48,12 +48,17 @@ class MetropolisExchangeSpinfulSamplerGPU(SamplerGPU):
         """n_sweeps sweeps in place (model.mcmc_sweep runs them in libvmcx);
         returns (sign, log|psi|) of the walkers afterwards."""
         edges = graph.edge_tensor(fxs.device, "sweep")
-        sign, logabs, n_acc = model.mcmc_sweep(fxs, edges, 0, self.seed, self.sweep_counter,
-                                               self.hopping_rate, self.refresh_every)
-        acc0 = n_acc.clone()
-        sign, logabs, n_acc = model.mcmc_sweep(fxs, edges, n_sweeps, self.seed,
-                                               self.sweep_counter, self.hopping_rate,
-                                               self.refresh_every, draws=draws)
+        # the parameters are constant over the call: looked at once, on entry
+        frozen = model.frozen() if hasattr(model, "frozen") else contextlib.nullcontext()
+        with frozen:
+            if hasattr(model, "accept_counts"):
+                acc0 = model.accept_counts(fxs).clone()
+            else:
+                acc0 = model.mcmc_sweep(fxs, edges, 0, self.seed, self.sweep_counter,
+                                        self.hopping_rate, self.refresh_every)[2].clone()
+            sign, logabs, n_acc = model.mcmc_sweep(fxs, edges, n_sweeps, self.seed,
+                                                   self.sweep_counter, self.hopping_rate,
+                                                   self.refresh_every, draws=draws)
         self.sweep_counter += n_sweeps
         if n_sweeps:
             self.last_acceptance = (n_acc - acc0, n_sweeps * edges.shape[0])

@@ -69,12 +69,22 @@ def check_grads_amps(O, sign, logabs, configs=None):
     reduction per tensor and one host read).  An amplitude is its sign and
     ln|psi|; ln|psi| = -inf is a zero amplitude, which the log form clamps
     to ln(1e-45), so any non-finite value is an error."""
-    bad_amp = ~(torch.isfinite(sign) & torch.isfinite(logabs))
-    # a NaN or Inf anywhere in a row makes its sum non-finite; the row sums
-    # avoid a full-size boolean temporary of O
-    bad_o = ~torch.isfinite(O.sum(dim=1)) if O.numel() else torch.zeros_like(bad_amp)
-    counts = torch.stack([bad_amp.sum(), bad_o.sum()]).cpu()
+    if (O.is_cuda and O.dtype in (torch.float64, torch.float32) and O.dim() == 2
+            and O.stride(1) == 1 and O.stride(0) >= O.shape[1]
+            and all(v.is_cuda and v.dtype == torch.float64 and v.is_contiguous()
+                    and v.shape == O.shape[:1] for v in (sign, logabs))):
+        # one pass over O, one host read
+        counts = kernels.count_nonfinite(O, sign, logabs).cpu()
+        bad_amp = None
+    else:
+        bad_amp = ~(torch.isfinite(sign) & torch.isfinite(logabs))
+        # a NaN or Inf anywhere in a row makes its sum non-finite; the row sums
+        # avoid a full-size boolean temporary of O
+        bad_o = ~torch.isfinite(O.sum(dim=1)) if O.numel() else torch.zeros_like(bad_amp)
+        counts = torch.stack([bad_amp.sum(), bad_o.sum()]).cpu()
     if int(counts[0]):
+        if bad_amp is None:
+            bad_amp = ~(torch.isfinite(sign) & torch.isfinite(logabs))
         idx = bad_amp.nonzero()[:20, 0].tolist()
         where = "" if configs is None else "; first configs: " + "; ".join(
             str(configs[i].tolist()) for i in idx)

@@ -52,6 +52,13 @@ constexpr int BMAX_SWEEPS = 30;
 // this floor are not rotated away (singular values below ~1e-9 of the
 // largest, which move an amplitude by about that much relative)
 constexpr double BM_ROT_FLOOR = 1e-18;
+// the pivoted Cholesky stops when the largest remaining diagonal entry is below this:
+// graded states (bond entries that fall off by 10 per index) need the small singular
+// values, which the factor and one-sided Jacobi keep to relative accuracy.  Against the
+// QR / SVD truncation, median relative error of an amplitude of such a 6x6 D = 4 chi = 8
+// state: 3e-8 with a floor of 4.4e-16, 3e-10 with 1e-18, 6e-11 with 1e-24 and below
+// (7e-10 with two-sided Jacobi); the floors cost the same time from 1e-18 on
+constexpr double BM_PIVOT_FLOOR = 1e-30;
 // int64 header words per boundary buffer: [0] log scale (double bits),
 // [1 .. Ly+1] bond dimensions, [Ly+2 .. 2Ly+2] bond parity masks
 constexpr int BHDR = 40;
@@ -282,12 +289,13 @@ __device__ __forceinline__ double bm_rsqrt(double x) {
 // orthonormal to FP64.  Measured on 6x6 D = 4 chi = 8, per 32 x 32 eigensolve with four
 // workgroups on a CU: 80 k cycles; 198 k on the columns of the block itself, and 1754 us
 // per launch of 2048 workgroups with two-sided Jacobi in LDS against 1020 us with this.
-// Columns are orthogonal to 4e-15 of their own norms; eigenvalues
-// below 1e-18 of the largest diagonal entry come out as zero vectors.
+// Columns are orthogonal to 4e-15 of their own norms; what the
+// factorisation leaves out (BM_PIVOT_FLOOR) comes out as zero vectors.
 // row: LDS scratch of 4 RPL doubles per block.
 // Output, compacted: columns off .. off + m of T (rows off .. off + m) and lam; the
-// caller has zeroed both.
-template <int JB, int RPL>
+// caller has zeroed both, or (CLEAR, JB = 3, off = 0, 16 x ld each) they are zeroed here
+// once R, which T may then be, is in registers.
+template <int JB, int RPL, bool CLEAR = false>
 __device__ __forceinline__ void bm_jacobi_wave(const double *R, int ld, int off, int m, int mmax, double *row,
                                double *T, double *lam) {
   constexpr int NJ = 1 << JB;   // columns j and j + NJ
@@ -313,8 +321,8 @@ __device__ __forceinline__ void bm_jacobi_wave(const double *R, int ld, int off,
     constexpr unsigned IM = 2 * NJ - 1;
     for (int step = 0; step < mmax; ++step) {
       // largest remaining diagonal entry (to FP32 precision, the column in the low bits)
-      const unsigned kt = dt > 1e-18 ? (__float_as_uint((float)dt) & ~IM) | c0 : 0u;
-      const unsigned kb = db > 1e-18 ? (__float_as_uint((float)db) & ~IM) | c1 : 0u;
+      const unsigned kt = dt > BM_PIVOT_FLOOR ? (__float_as_uint((float)dt) & ~IM) | c0 : 0u;
+      const unsigned kb = db > BM_PIVOT_FLOOR ? (__float_as_uint((float)db) & ~IM) | c1 : 0u;
       unsigned key = kt > kb ? kt : kb;
       key = max(key, (unsigned)bm_xor32<1>((int)key));
       key = max(key, (unsigned)bm_xor32<2>((int)key));
@@ -348,6 +356,11 @@ __device__ __forceinline__ void bm_jacobi_wave(const double *R, int ld, int off,
       db = c1 == q ? 0.0 : fma(-lb, lb, db);
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
+  }
+  if constexpr (CLEAR) {
+    for (int i = lane & 31; i < 16 * ld; i += 32) T[i] = 0.0;
+    if ((lane & 31) < 16) lam[lane & 31] = 0.0;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   }
   // columns 0 .. rank - 1 are set: pairs over the first G0 lanes
   int G0 = 1;
@@ -1092,6 +1105,589 @@ __global__ void __launch_bounds__(BT, NB == 32 ? 4 : 1)
     for (int i = start; i < nrows; ++i) hd[i * bufd * BHDR] = __double_as_longlong(-INFINITY);
 }
 
+// ------------------------------------------------------------ one side, one wave
+// The same side in one wave with the dense products on v_mfma_f64_16x16x4f64, for bonds
+// whose Z2 sectors hold at most 16 absorbed indices (bm_wave_fits).  Lane l, register r of
+// a result holds D[4 r + l / 16][l % 16]; k-step r of an operand holds A[l % 16][4 r + l / 16]
+// and B[4 r + l / 16][l % 16], so a result read as the A operand is its transpose.
+//
+// Absorbed bond indices (a, l) are numbered within their sector.  The block (s, c) of
+// A_v[(a,l)][(b,r)] is nonzero for v of one parity, so number t of the even and of the odd
+// v make one operand F (p64-style pairs: two at D = 4, one at D = 2), whose fragments each
+// lane forms from B and the slice (two of the u are nonzero).  Then, per block (s, c):
+//   T^T = R_c F^T  (R_c symmetric: a result serves as the A operand),
+//   R'_s += T F^T  (T^T as a result is T as the A operand; F^T as before),
+// so the Grams stay in registers from the last column to the first; each is also stored
+// for the way back.  There C = sum P F, rho_s = C R C^T by the same two steps, its
+// eigenvectors (bm_jacobi_wave, both sectors), P' = U^T C.
+//
+// Bound by the latency of one wave's chain; the workgroup-per-side kernel kept three of
+// four waves idle in the eigensolver, read two LDS operands per multiply-add in the
+// products and did four times as many (the zero blocks).  LDS 12 KB: up to 13 waves on a
+// CU instead of 4 sides.  6x6 D = 4 chi = 8, 1024 walkers: sampling phase 133.8 ->
+// 48.4 ms (with the join below; 52.6 and 60.1 ms when held to 168 and 128 registers).
+constexpr int BWL = 17;   // LDS row stride of the 16 x 16 blocks
+
+bool bm_wave_fits(int D, int cb) {
+  const int sector = D == 3 ? 2 * cb : D * cb / 2;
+  return D >= 2 && sector <= 16;
+}
+
+// number t of the even (odd = 0) or odd values of a leg of dimension D; -1: none
+template <int D>
+__device__ __forceinline__ int bm_leg(int odd, int t) {
+  constexpr int ne = D >> 1;
+  const int v = odd ? ne + t : t;
+  return (odd ? v < D : t < ne) ? v : -1;
+}
+
+struct BmWaveSh {
+  double Sl[256];            // slice [l][f][o][r]
+  double U[2][16 * BWL];     // rho, then its eigenvectors; P [16][33] until the next C
+  double C[2][16 * BWL];     // by sector of (k, v)
+  double lam[32], row[32];
+  int perm[2][32];           // left / right bond: sector 16 + number -> a | l << 8 | par(a) << 16
+  int kv[32];                // (k, v) -> sector << 8 | number
+  int sel[32];
+};
+
+__device__ __forceinline__ void bm_wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+__device__ __forceinline__ double bm_wave_max(double v) {
+  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
+  return v;
+}
+
+typedef double bmd4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ bmd4 bm_mfma4(const double (&a)[4], const double (&b)[4], bmd4 acc) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a[r], b[r], acc, 0, 0, 0);
+  return acc;
+}
+
+template <int D>
+__global__ void __launch_bounds__(64, 2)
+    peps_bmps_wave_kernel(BmGeo g, int64_t rows, const int64_t *__restrict__ cfg,
+                          const int32_t *__restrict__ flag, double *ws, int64_t *hdr, int st_top,
+                          int st_bot, const double *__restrict__ cache,
+                          const int64_t *__restrict__ chdr, const int32_t *__restrict__ parent,
+                          const uint32_t *__restrict__ cmove) {
+  constexpr int NPAIR = D > 2 ? 2 : 1;      // pairs of an even and an odd leg value
+  const int64_t w = blockIdx.x;
+  if (w >= rows) return;
+  if (flag && !(flag[w] & 1)) return;
+  const int side = blockIdx.y;
+  const bool down = side == 0;
+  const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
+  if (cache && cmove) bm_move_starts(g, cmove[w], st_top, st_bot);
+  const int start = cache ? (down ? st_top : st_bot) : 0;
+  const int64_t pw = parent ? (int64_t)parent[w] : w;
+  const int Ly = g.Ly, h = g.Lx / 2, cb = g.cb;
+  const int nrows = (g.nbuf > 1 && !g.half) ? g.Lx - 1 : (down ? h : g.Lx - h);
+  if (start >= nrows) return;
+  __shared__ BmWaveSh S;
+  const double *th = g.theta + w * g.theta_stride;
+  double *slot = ws + (w * 2 + side) * g.slot;
+  const int64_t bstride = (int64_t)Ly * g.ts;
+  double *Rg = slot + g.nbuf * bstride;       // [y][sector][register][lane]
+  int64_t *hd = hdr + (w * 2 + side) * g.nbuf * BHDR;
+  const int bufd = g.nbuf > 1 ? 1 : 0;
+  const double *cslot = cache ? cache + (pw * 2 + side) * g.slot : nullptr;
+  const int64_t *chd = chdr ? chdr + (pw * 2 + side) * g.nbuf * BHDR : nullptr;
+
+  // the configuration as bit masks; lane s: dense offset of site s
+  const int code = lane < g.N ? (int)cfg[w * g.N + lane] : 0;
+  const uint64_t dn = __ballot(code & 1), up = __ballot(code & 2), sing = dn ^ up;
+  int doff;
+  {
+    const int x = lane / Ly, y = lane - x * Ly;
+    const int n = lane < g.N ? 4 * (y == 0 ? 1 : D) * (x == 0 ? 1 : D) *
+                                   (x == g.Lx - 1 ? 1 : D) * (y == Ly - 1 ? 1 : D)
+                             : 0;
+    int sum = n;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int t = __shfl_up(sum, o);
+      if (lane >= o) sum += t;
+    }
+    doff = sum - n;
+  }
+  auto site_par = [&](int x, int y) { return (int)((sing >> (x * Ly + y)) & 1); };
+  auto leg = [&](int y) { return (y == 0 || y == Ly) ? 1 : D; };   // horizontal bond y
+  // signed slice of site (x, y): entries lane, lane + 64, ... in registers
+  auto fetch = [&](int x, int y, double (&sv)[4]) {
+    const int s = x * Ly + y;
+    const int dl = leg(y), dr = leg(y + 1), du = x == 0 ? 1 : D, dd = x == g.Lx - 1 ? 1 : D;
+    const int n = dl * du * dd * dr;
+    const int p = (int)((dn >> s) & 1) | ((int)((up >> s) & 1) << 1);
+    const uint64_t right = s + 1 < 64 ? (sing >> (s + 1)) & ((1ull << (Ly - 1 - y)) - 1) : 0;
+    const int pr = __popcll(right) & 1;
+    const int base = __builtin_amdgcn_readlane(doff, s) + p * n;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int idx = lane + 64 * q;
+      const int r = dr == 1 ? 0 : idx % D, i1 = dr == 1 ? idx : idx / D;
+      const int d = dd == 1 ? 0 : i1 % D;
+      const int k = idx < n ? g.dmap[base + idx] : -1;
+      double v = k >= 0 ? th[k] : 0.0;
+      if ((bqpar(d, dd) * (bqpar(r, dr) + pr)) & 1) v = -v;
+      sv[q] = v;
+    }
+  };
+  // ... into LDS as [l][f][o][r] (f: the leg facing the boundary)
+  auto stash = [&](int x, int y, const double (&sv)[4]) {
+    const int dl = leg(y), dr = leg(y + 1), du = x == 0 ? 1 : D, dd = x == g.Lx - 1 ? 1 : D;
+    const int n = dl * du * dd * dr;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int idx = lane + 64 * q;
+      if (idx >= n) continue;
+      int to = idx;
+      if (!down) {
+        const int r = dr == 1 ? 0 : idx % D, i1 = dr == 1 ? idx : idx / D;
+        const int d = dd == 1 ? 0 : i1 % D, i2 = dd == 1 ? i1 : i1 / D;
+        const int u = du == 1 ? 0 : i2 % D, l = du == 1 ? i2 : i2 / D;
+        to = ((l * dd + d) * du + u) * dr + r;
+      }
+      S.Sl[to] = sv[q];
+    }
+  };
+
+  double lg = 0.0;
+  bool dead = false;
+  // lane y: dimension and parity mask of bond y; cm: bit y = parity of the nonzero
+  // entries of B_y
+  int bd = 1, bpm = 0, cm = 0;
+  constexpr int dmask = ((1 << D) - 1) & ~((1 << (D >> 1)) - 1);
+  if (start > 0) {
+    const int64_t *c = chd + (start - 1) * bufd * BHDR;
+    if (lane <= Ly) {
+      bd = (int)c[1 + lane];
+      bpm = (int)c[Ly + 2 + lane];
+    }
+    cm = __builtin_amdgcn_readfirstlane((int)c[2 * Ly + 3]);
+    lg = __longlong_as_double(c[0]);
+    dead = std::isinf(lg);
+  } else if (lane <= Ly) {
+    bd = leg(lane);
+    bpm = bd == 1 ? 0 : dmask;
+  }
+  auto write_header = [&](int64_t *to) {
+    if (lane <= Ly) {
+      to[1 + lane] = bd;
+      to[Ly + 2 + lane] = (int64_t)bpm;
+    }
+    if (lane == 0) {
+      to[0] = __double_as_longlong(dead ? -INFINITY : lg);
+      to[2 * Ly + 3] = cm;
+    }
+  };
+  // tensor entries v[q] at offsets to[q] (-1: none) scaled by 1 / max; false: a zero tensor
+  auto store_scaled = [&](double *dst, const double (&v)[8], const int (&to)[8]) {
+    double m = 0.0;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) m = fmax(m, to[q] >= 0 ? fabs(v[q]) : 0.0);
+    m = bm_wave_max(m);
+    if (!(m > 0.0) || !std::isfinite(m)) return false;
+    const double inv = 1.0 / m;
+#pragma unroll
+    for (int q = 0; q < 8; ++q)
+      if (to[q] >= 0) dst[to[q]] = v[q] * inv;
+    lg += log(m);
+    return true;
+  };
+  // first row: B_y[l][v][r] = S[l][0][v][r]
+  if (start == 0) {
+    const int x = down ? 0 : g.Lx - 1;
+    for (int y = 0; y < Ly && !dead; ++y) {
+      double sv[4];
+      fetch(x, y, sv);
+      const int dl = leg(y), dr = leg(y + 1), n = dl * D * dr;
+      // the facing leg has dimension 1: [l][v][r] whichever side
+      double v[8] = {sv[0], 0, 0, 0, 0, 0, 0, 0};
+      int to[8] = {lane < n ? (dr == 1 ? lane : lane / D) * cb + (dr == 1 ? 0 : lane % D) : -1,
+                   -1, -1, -1, -1, -1, -1, -1};
+      if (!store_scaled(slot + (int64_t)y * g.ts, v, to)) dead = true;
+      cm |= site_par(x, y) << y;
+    }
+    write_header(hd);
+  }
+  for (int ri = start > 1 ? start : 1; ri < nrows && !dead; ++ri) {
+    const int x = down ? ri : g.Lx - 1 - ri;
+    const double *src = (start > 0 && ri == start) ? cslot + (ri - 1) * bstride
+                                                   : slot + (ri - 1) * bufd * bstride;
+    double *dst = slot + ri * bufd * bstride;
+    bm_wave_fence();   // the last row's tensors are this row's
+    double sv[4], svn[4];
+    if (__ballot(lane <= Ly && bd * leg(lane) > g.chi) == 0) {
+      // absorb without truncation
+      for (int y = 0; y < Ly && !dead; ++y) {
+        fetch(x, y, sv);
+        stash(x, y, sv);
+        bm_wave_fence();
+        const int na = __builtin_amdgcn_readlane(bd, y), nb = __builtin_amdgcn_readlane(bd, y + 1);
+        const int dl = leg(y), dr = leg(y + 1), nj = nb * dr, n = na * dl * D * nj;
+        const double *B = src + (int64_t)y * g.ts;
+        double v[8];
+        int to[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int idx = lane + 64 * q;
+          v[q] = 0.0;
+          to[q] = -1;
+          if (idx < n) {
+            const int j = idx % nj, iv = idx / nj, vv = iv % D, i = iv / D;
+            const int a = dl == 1 ? i : i / D, l = dl == 1 ? 0 : i % D;
+            const int b = dr == 1 ? j : j / D, r = dr == 1 ? 0 : j % D;
+            double t = 0.0;
+#pragma unroll
+            for (int u = 0; u < D; ++u)
+              t = fma(B[(a * D + u) * cb + b], S.Sl[((l * D + u) * D + vv) * dr + r], t);
+            v[q] = t;
+            to[q] = iv * cb + j;
+          }
+        }
+        if (!store_scaled(dst + (int64_t)y * g.ts, v, to)) dead = true;
+        bm_wave_fence();
+        cm ^= site_par(x, y) << y;
+      }
+      const int hdy = lane <= Ly ? leg(lane) : 1;
+      int m = 0;
+      for (int a = 0; a < bd; ++a)
+        for (int l = 0; l < hdy; ++l)
+          if (((bpm >> a) & 1) ^ bqpar(l, hdy)) m |= 1 << (a * hdy + l);
+      bd *= hdy;
+      bpm = m;
+      write_header(hd + ri * bufd * BHDR);
+      continue;
+    }
+    // sector numbering of absorbed bond y into perm[o]
+    auto number_bond = [&](int y, int o) {
+      const int nb = __builtin_amdgcn_readlane(bd, y), mk = __builtin_amdgcn_readlane(bpm, y);
+      const int hdy = leg(y), n = nb * hdy;
+      const int a = hdy == 1 ? lane : lane / D, l = hdy == 1 ? 0 : lane % D;
+      const int pa = (mk >> (a & 31)) & 1, par = pa ^ bqpar(l, hdy);
+      const uint64_t odd = __ballot(lane < n && par), even = __ballot(lane < n && !par);
+      const int num = __popcll((par ? odd : even) & ((1ull << lane) - 1));
+      if (lane < 32) S.perm[o][lane] = -1;
+      bm_wave_fence();
+      if (lane < n) S.perm[o][par * 16 + num] = a | (l << 8) | (pa << 16);
+      bm_wave_fence();
+    };
+    // B[a][u][b] of the two nonzero u of an entry (left code, right code), and the entry of
+    // A_v from them
+    auto b_entry = [&](const double *B, int cy, int lc, int rc, double (&bv)[2]) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const int u = bm_leg<D>(cy ^ ((lc >> 16) & 1) ^ ((rc >> 16) & 1), q);
+        bv[q] = (q < NPAIR && (lc | rc) >= 0 && u >= 0)
+                    ? B[((lc & 255) * D + u) * cb + (rc & 255)]
+                    : 0.0;
+      }
+    };
+    auto a_entry = [&](int cy, int lc, int rc, const double (&bv)[2], int v, int dr) {
+      double t = 0.0;
+      if (v >= 0 && (lc | rc) >= 0)
+#pragma unroll
+        for (int q = 0; q < NPAIR; ++q) {
+          const int u = bm_leg<D>(cy ^ ((lc >> 16) & 1) ^ ((rc >> 16) & 1), q);
+          if (u >= 0)
+            t = fma(bv[q], S.Sl[((((lc >> 8) & 255) * D + u) * D + v) * dr + ((rc >> 8) & 255)], t);
+        }
+      return t;
+    };
+    // ---- right Grams, y = Ly-1 .. 1 (R_Ly = 1 at the even index 0)
+    double R[2][4] = {{lane == 0 ? 1.0 : 0.0, 0, 0, 0}, {0, 0, 0, 0}};
+    fetch(x, Ly - 1, sv);
+    number_bond(Ly, 1);
+    for (int y = Ly - 1; y >= 1; --y) {
+      const int lo = (Ly - 1 - y) & 1, ro = lo ^ 1;   // perm buffers of the left and right bond
+      number_bond(y, lo);
+      stash(x, y, sv);
+      bm_wave_fence();
+      fetch(x, y > 1 ? y - 1 : 0, svn);
+      const int cy = (cm >> y) & 1, ey = cy ^ site_par(x, y), dr = leg(y + 1);
+      const double *B = src + (int64_t)y * g.ts;
+      bmd4 acc[2] = {{0, 0, 0, 0}, {0, 0, 0, 0}};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const int lc = S.perm[lo][s * 16 + li];
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+          double bv[4][2];
+          int rc[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            rc[r] = S.perm[ro][c * 16 + 4 * r + lk];
+            b_entry(B, cy, lc, rc[r], bv[r]);
+          }
+#pragma unroll
+          for (int t = 0; t < NPAIR; ++t) {
+            const int v = bm_leg<D>(ey ^ s ^ c, t);
+            if (v < 0) continue;
+            double F[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) F[r] = a_entry(cy, lc, rc[r], bv[r], v, dr);
+            const bmd4 z = {0, 0, 0, 0};
+            const bmd4 tt = bm_mfma4(R[c], F, z);
+            const double T[4] = {tt[0], tt[1], tt[2], tt[3]};
+            acc[s] = bm_mfma4(T, F, acc[s]);
+          }
+        }
+      }
+      double mx = 0.0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) mx = fmax(mx, fmax(fabs(acc[0][r]), fabs(acc[1][r])));
+      mx = bm_wave_max(mx);
+      const double inv = mx > 0.0 ? 1.0 / mx : 0.0;
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          R[s][r] = acc[s][r] * inv;
+          Rg[(((int64_t)y * 2 + s) * 4 + r) * 64 + lane] = R[s][r];
+        }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sv[q] = svn[q];
+      bm_wave_fence();
+    }
+    // ---- forward: truncation left to right
+    double *P = &S.U[0][0];
+    constexpr int PLD = 33;
+    for (int i = lane; i < 16 * PLD; i += 64) P[i] = 0.0;
+    int k = 1, kp = 0, E = 0;        // kept bond: dimension, parity mask; parity so far
+    int nbd = lane == 0 ? 1 : 0, npm = 0;
+    bm_wave_fence();
+    if (lane == 0) P[0] = 1.0;
+    fetch(x, 0, sv);
+    number_bond(0, 0);
+    for (int y = 0; y < Ly && !dead; ++y) {
+      const int lo = y & 1, ro = lo ^ 1;
+      number_bond(y + 1, ro);
+      stash(x, y, sv);
+      const int nC = k * D;
+      int nkv[2];
+      {
+        const int kk = lane / D, v = lane % D;
+        const int par = ((kp >> (kk & 31)) & 1) ^ bqpar(v, D);
+        const uint64_t odd = __ballot(lane < nC && par), even = __ballot(lane < nC && !par);
+        nkv[0] = __popcll(even);
+        nkv[1] = __popcll(odd);
+        if (lane < nC) S.kv[lane] = (par << 8) | __popcll((par ? odd : even) & ((1ull << lane) - 1));
+      }
+      for (int i = lane; i < 2 * 16 * BWL; i += 64) (&S.C[0][0])[i] = 0.0;
+      bm_wave_fence();
+      fetch(x, y + 1 < Ly ? y + 1 : y, svn);
+      const int cy = (cm >> y) & 1, ey = cy ^ site_par(x, y), dr = leg(y + 1);
+      const int E2 = E ^ ey;
+      const double *B = src + (int64_t)y * g.ts;
+      // C[(k,v)][(b,r)] = sum_{(a,l)} P[k][(a,l)] A_v[(a,l)][(b,r)]: the row k of the
+      // product has its (a,l) in sector par(k) ^ E, hence one v per pair
+      double Pf[2][4];
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) Pf[s][r] = P[li * PLD + s * 16 + 4 * r + lk];
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        bmd4 acc[NPAIR];
+#pragma unroll
+        for (int t = 0; t < NPAIR; ++t) acc[t] = (bmd4){0, 0, 0, 0};
+        const int rc = S.perm[ro][c * 16 + li];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          double bv[4][2];
+          int lc[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            lc[r] = S.perm[lo][s * 16 + 4 * r + lk];
+            b_entry(B, cy, lc[r], rc, bv[r]);
+          }
+#pragma unroll
+          for (int t = 0; t < NPAIR; ++t) {
+            const int v = bm_leg<D>(ey ^ s ^ c, t);
+            if (v < 0) continue;
+            double F[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) F[r] = a_entry(cy, lc[r], rc, bv[r], v, dr);
+            acc[t] = bm_mfma4(Pf[s], F, acc[t]);
+          }
+        }
+        // rows (k, v) of the sector that belongs to column sector c
+#pragma unroll
+        for (int t = 0; t < NPAIR; ++t)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kk = 4 * r + lk;
+            const int v = bm_leg<D>(E2 ^ c ^ ((kp >> kk) & 1), t);
+            if (kk < k && v >= 0) {
+              const int at = S.kv[kk * D + v];
+              S.C[at >> 8][(at & 255) * BWL + li] = acc[t][r];
+            }
+          }
+      }
+      bm_wave_fence();
+      if (y == Ly - 1) {
+        // last site: B'[k][v][0] = C[(k,v)][0]
+        double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        int to[8] = {-1, -1, -1, -1, -1, -1, -1, -1};
+        if (lane < nC) {
+          const int at = S.kv[lane];
+          v[0] = S.C[at >> 8][(at & 255) * BWL];
+          // the other sector's only nonzero column is not this one
+          if ((at >> 8) != E2) v[0] = 0.0;
+          to[0] = lane * cb;
+        }
+        if (!store_scaled(dst + (int64_t)y * g.ts, v, to)) dead = true;
+        if (lane == Ly) {
+          nbd = 1;
+          npm = 0;
+        }
+        cm = E2 << (Ly - 1);
+        break;
+      }
+      double *dsty = dst + (int64_t)y * g.ts;
+      int kn, kpn;
+      double pm = 0.0;
+      if (nC <= g.chi) {
+        // no truncation at this bond: the identity basis, P = C
+        kn = nC;
+        const int at0 = lane < nC ? S.kv[lane] : 0;
+        kpn = (int)__ballot(lane < nC && (at0 >> 8));
+        for (int idx = lane; idx < nC * kn; idx += 64) {
+          const int j = idx % kn, kv = idx / kn;
+          dsty[kv * cb + j] = j == kv ? 1.0 : 0.0;
+        }
+        double v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          // entry (row kv, position) of P: kv = (lane + 64 q) / 32
+          const int idx = lane + 64 * q, kv = idx >> 5, pos = idx & 31;
+          v[q] = 0.0;
+          if (kv < nC) {
+            const int at = S.kv[kv];
+            if (((at >> 8) ^ E2) == (pos >> 4)) v[q] = S.C[at >> 8][(at & 255) * BWL + (pos & 15)];
+          }
+          pm = fmax(pm, fabs(v[q]));
+        }
+        pm = bm_wave_max(pm);
+        const double pinv = 1.0 / pm;
+        if (pm > 0.0)
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            const int idx = lane + 64 * q;
+            P[(idx >> 5) * PLD + (idx & 31)] = v[q] * pinv;
+          }
+      } else {
+        kn = g.chi;
+        // rho_s = C_s R C_s^T
+        bmd4 rho[2];
+        double dmx = 0.0;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          double Rf[4], Cf[4];
+          const double *Rs = Rg + ((int64_t)(y + 1) * 2 + (s ^ E2)) * 256;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            Rf[r] = Rs[r * 64 + lane];
+            Cf[r] = S.C[s][li * BWL + 4 * r + lk];
+          }
+          const bmd4 z = {0, 0, 0, 0};
+          const bmd4 tt = bm_mfma4(Rf, Cf, z);
+          const double T[4] = {tt[0], tt[1], tt[2], tt[3]};
+          rho[s] = bm_mfma4(T, Cf, z);
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (4 * r + lk == li) dmx = fmax(dmx, fabs(rho[s][r]));
+        }
+        dmx = bm_wave_max(dmx);
+        if (!(dmx > 0.0)) {
+          dead = true;
+          break;
+        }
+        const double dinv = 1.0 / dmx;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) S.U[s][(4 * r + lk) * BWL + li] = rho[s][r] * dinv;
+        bm_wave_fence();
+        const int hs = lane >> 5;
+        bm_jacobi_wave<3, 4, true>(S.U[hs], BWL, 0, hs ? nkv[1] : nkv[0], nkv[0] > nkv[1] ? nkv[0] : nkv[1],
+                                   S.row + 16 * hs, S.U[hs], S.lam + 16 * hs);
+        bm_wave_fence();
+        // the chi leading eigenvalues: column (sector, number) = lane
+        const double lam = (lane < 32 && li < (lk ? nkv[1] : nkv[0])) ? S.lam[lane] : -1.0;
+        int rank = 0;
+#pragma unroll
+        for (int q = 0; q < 32; ++q) {
+          const double lq = __shfl(lam, q);
+          rank += (lq > lam) || (lq == lam && q < lane);
+        }
+        const int rk = (lane < 32 && lam >= 0.0 && rank < kn) ? rank : -1;
+        if (rk >= 0) S.sel[rk] = lane;
+        bm_wave_fence();
+        kpn = (int)__ballot(lane < kn && (S.sel[lane & 31] >> 4));
+        for (int idx = lane; idx < nC * kn; idx += 64) {
+          const int j = idx % kn, kv = idx / kn, at = S.kv[kv], sj = S.sel[j];
+          dsty[kv * cb + j] = (at >> 8) == (sj >> 4) ? S.U[at >> 8][(at & 255) * BWL + (sj & 15)] : 0.0;
+        }
+        // P' = U^T C: all columns of a sector at once, the chosen ones kept
+        bmd4 pn[2];
+        int to[2][4];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          double Uf[4], Cf[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            Uf[r] = S.U[s][(4 * r + lk) * BWL + li];
+            Cf[r] = S.C[s][(4 * r + lk) * BWL + li];
+          }
+          const bmd4 z = {0, 0, 0, 0};
+          pn[s] = bm_mfma4(Uf, Cf, z);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            to[s][r] = __shfl(rk, s * 16 + 4 * r + lk);
+            if (to[s][r] >= 0) pm = fmax(pm, fabs(pn[s][r]));
+          }
+        }
+        pm = bm_wave_max(pm);
+        bm_wave_fence();
+        for (int i = lane; i < 16 * PLD; i += 64) P[i] = 0.0;
+        bm_wave_fence();
+        const double pinv = 1.0 / pm;
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (to[s][r] >= 0) P[to[s][r] * PLD + (s ^ E2) * 16 + li] = pn[s][r] * pinv;
+      }
+      if (!(pm > 0.0) || !std::isfinite(pm)) {
+        dead = true;
+        break;
+      }
+      lg += log(pm);
+      if (lane == y + 1) {
+        nbd = kn;
+        npm = kpn;
+      }
+      k = kn;
+      kp = kpn;
+      E = E2;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) sv[q] = svn[q];
+      bm_wave_fence();
+    }
+    bd = nbd;
+    bpm = npm;
+    write_header(hd + ri * bufd * BHDR);
+  }
+  // buffers never reached (a vanishing boundary): mark them zero
+  if (dead && lane == 0)
+    for (int i = start; i < nrows; ++i) hd[i * bufd * BHDR] = __double_as_longlong(-INFINITY);
+}
+
 // ------------------------------------------------------------ join
 // the amplitude from the top boundary in buffer bt and the bottom one in bb
 __global__ void __launch_bounds__(64)
@@ -1182,6 +1778,119 @@ __global__ void __launch_bounds__(64)
   }
   if (tid == 0) {
     const double v = E[0] * (((P * (P - 1) / 2) & 1) ? -1.0 : 1.0);
+    if (v == 0.0 || !std::isfinite(v)) {
+      sign[w] = 0.0;
+      logabs[w] = lo;
+    } else {
+      sign[w] = v > 0.0 ? 1.0 : -1.0;
+      logabs[w] = fmax(log(fabs(v)) + lsc + lt + lb, lo);
+    }
+  }
+}
+
+// The same join for bonds of at most 16, on v_mfma_f64_16x16x4f64 with everything in
+// registers (layouts as in peps_bmps_wave_kernel): X_v = E^T T_v and E' += X_v^T Bo_v, each
+// result being the next product's A operand; the next site's tensors are loaded during the
+// products.  Bound by the latency of a wave's chain of Ly sites: 18 us for 1024
+// configurations of 6x6 D = 4 chi = 8; over the calls of a sampling phase 31 us on average
+// against 103 us with E and X in LDS.
+template <int D>
+__global__ void __launch_bounds__(64)
+    peps_bmps_join_wave_kernel(BmGeo g, int64_t rows, const int64_t *__restrict__ cfg,
+                               const int32_t *__restrict__ flag, const double *__restrict__ ws,
+                               const int64_t *__restrict__ hdr, int bt, int bb, double *sign,
+                               double *logabs, int ct, int cb_, const double *__restrict__ cache,
+                               const int64_t *__restrict__ chdr,
+                               const int32_t *__restrict__ parent,
+                               const uint32_t *__restrict__ cmove) {
+  const int64_t w = blockIdx.x;
+  if (w >= rows) return;
+  if (flag && !(flag[w] & 1)) return;
+  const int lane = threadIdx.x, li = lane & 15, lk = lane >> 4;
+  if (cache && cmove) {
+    int s0, s1;
+    bm_move_starts(g, cmove[w], s0, s1);
+    ct = s0 >= g.Lx / 2;
+    cb_ = s1 >= g.Lx - g.Lx / 2;
+  }
+  const int64_t pw = parent ? (int64_t)parent[w] : w;
+  const int64_t *ht = ct ? chdr + ((pw * 2) * g.nbuf + bt) * BHDR
+                         : hdr + ((w * 2) * g.nbuf + bt) * BHDR;
+  const int64_t *hb = cb_ ? chdr + ((pw * 2 + 1) * g.nbuf + bb) * BHDR
+                          : hdr + ((w * 2 + 1) * g.nbuf + bb) * BHDR;
+  const double lt = __longlong_as_double(ht[0]), lb = __longlong_as_double(hb[0]);
+  const double lo = log(1e-45);
+  const int code = lane < g.N ? (int)cfg[w * g.N + lane] : 0;
+  const int P = __popcll(__ballot(code == 1 || code == 2));
+  const int64_t bstride = (int64_t)g.Ly * g.ts;
+  const double *Tt = ct ? cache + (pw * 2) * g.slot + bt * bstride
+                        : ws + (w * 2) * g.slot + bt * bstride;
+  const double *Tb = cb_ ? cache + (pw * 2 + 1) * g.slot + bb * bstride
+                         : ws + (w * 2 + 1) * g.slot + bb * bstride;
+  const int cb = g.cb, Ly = g.Ly;
+  bool zero = std::isinf(lt) || std::isinf(lb);
+  double e0 = 0.0, lsc = 0.0;
+  if (!zero) {
+    const int dt = lane <= Ly ? (int)ht[1 + lane] : 0, db = lane <= Ly ? (int)hb[1 + lane] : 0;
+    struct Ops {
+      double t[D][4], b[D][4];
+    };
+    auto load = [&](int y, Ops &o) {
+      const int ta = __builtin_amdgcn_readlane(dt, y), tb = __builtin_amdgcn_readlane(dt, y + 1);
+      const int ba = __builtin_amdgcn_readlane(db, y), bb2 = __builtin_amdgcn_readlane(db, y + 1);
+      const double *T = Tt + (int64_t)y * g.ts, *Bo = Tb + (int64_t)y * g.ts;
+#pragma unroll
+      for (int v = 0; v < D; ++v)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int a = 4 * r + lk;
+          o.t[v][r] = (a < ta && li < tb) ? T[(a * D + v) * cb + li] : 0.0;
+          o.b[v][r] = (a < ba && li < bb2) ? Bo[(a * D + v) * cb + li] : 0.0;
+        }
+    };
+    bmd4 E = {lane == 0 ? 1.0 : 0.0, 0.0, 0.0, 0.0};
+    Ops cur, nxt;
+    load(0, cur);
+    for (int y = 0; y < Ly; ++y) {
+      const int ta = __builtin_amdgcn_readlane(dt, y), ba = __builtin_amdgcn_readlane(db, y);
+      load(y + 1 < Ly ? y + 1 : y, nxt);
+      bmd4 X[D], out[2] = {{0.0, 0.0, 0.0, 0.0}, {0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+      for (int v = 0; v < D; ++v) X[v] = (bmd4){0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * r < ta)
+#pragma unroll
+          for (int v = 0; v < D; ++v)
+            X[v] = __builtin_amdgcn_mfma_f64_16x16x4f64(E[r], cur.t[v][r], X[v], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (4 * r < ba)
+#pragma unroll
+          for (int v = 0; v < D; ++v)
+            out[v & 1] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[v][r], cur.b[v][r], out[v & 1], 0,
+                                                              0, 0);
+      double mx = 0.0;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        E[r] = out[0][r] + out[1][r];
+        mx = fmax(mx, fabs(E[r]));
+      }
+      mx = bm_wave_max(mx);
+      if (!(mx > 0.0) || !std::isfinite(mx)) {
+        zero = true;
+        break;
+      }
+      const double inv = 1.0 / mx;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) E[r] *= inv;
+      lsc += log(mx);
+      cur = nxt;
+    }
+    e0 = E[0];
+  }
+  if (lane == 0) {
+    const double v = zero ? 0.0 : e0 * (((P * (P - 1) / 2) & 1) ? -1.0 : 1.0);
     if (v == 0.0 || !std::isfinite(v)) {
       sign[w] = 0.0;
       logabs[w] = lo;
@@ -1453,21 +2162,44 @@ BmGeo bm_geo(int Lx, int Ly, int D, int chi, int nbuf, int half = 0) {
   g.cb = chi > D ? chi : D;
   g.nbuf = nbuf;
   g.ts = (int64_t)g.cb * D * g.cb;
-  g.slot = (int64_t)nbuf * Ly * g.ts + (int64_t)Ly * BN * BN;
+  g.slot = (int64_t)nbuf * Ly * g.ts + (int64_t)Ly * (bm_wave_fits(D, g.cb) ? 512 : BN * BN);
   return g;
 }
-// the side kernel with 32 x 32 working matrices when chi * D allows (about
-// 45 KB of LDS, several workgroups per CU), else 64 x 64 (one per CU)
+// a wave per side when the sectors fit 16 x 16 blocks; else the workgroup kernel, with
+// 32 x 32 working matrices when chi * D allows (38 KB of LDS, several workgroups per CU)
+// or 64 x 64 (one per CU)
 void launch_side(const BmGeo &g, int64_t n, const int64_t *c, const int32_t *f, double *slots,
                  int64_t *hdr, hipStream_t st, int st_top = 0, int st_bot = 0,
                  const double *cache = nullptr, const int64_t *chdr = nullptr,
                  const int32_t *parent = nullptr, const uint32_t *cmove = nullptr) {
-  if (g.cb * g.D <= 32)
+  if (bm_wave_fits(g.D, g.cb)) {
+    const auto kern = g.D == 2   ? peps_bmps_wave_kernel<2>
+                      : g.D == 3 ? peps_bmps_wave_kernel<3>
+                                 : peps_bmps_wave_kernel<4>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)n, 2), dim3(64), 0, st, g, n, c, f, slots, hdr,
+                       st_top, st_bot, cache, chdr, parent, cmove);
+  } else if (g.cb * g.D <= 32)
     hipLaunchKernelGGL(peps_bmps_side_kernel<32>, dim3((unsigned)n, 2), dim3(BT), 0, st, g, n,
                        c, f, slots, hdr, st_top, st_bot, cache, chdr, parent, cmove);
   else
     hipLaunchKernelGGL(peps_bmps_side_kernel<64>, dim3((unsigned)n, 2), dim3(BT), 0, st, g, n,
                        c, f, slots, hdr, st_top, st_bot, cache, chdr, parent, cmove);
+}
+
+// (sign, ln|psi|) of n configurations from the boundaries in buffers bt and bb; one wave
+// each, on the matrix cores while the bonds fit one 16 x 16 tile
+void launch_join(const BmGeo &g, int64_t n, const int64_t *c, const int32_t *f,
+                 const double *slots, const int64_t *hdr, int bt, int bb, double *sign,
+                 double *logabs, hipStream_t st, int ct = 0, int cb = 0,
+                 const double *cache = nullptr, const int64_t *chdr = nullptr,
+                 const int32_t *parent = nullptr, const uint32_t *cmove = nullptr) {
+  const auto kern = g.cb > 16  ? peps_bmps_join_kernel
+                    : g.D == 1 ? peps_bmps_join_wave_kernel<1>
+                    : g.D == 2 ? peps_bmps_join_wave_kernel<2>
+                    : g.D == 3 ? peps_bmps_join_wave_kernel<3>
+                               : peps_bmps_join_wave_kernel<4>;
+  hipLaunchKernelGGL(kern, dim3((unsigned)n), dim3(64), 0, st, g, n, c, f, slots, hdr, bt, bb,
+                     sign, logabs, ct, cb, cache, chdr, parent, cmove);
 }
 }  // namespace
 
@@ -1508,9 +2240,7 @@ int bmps_amplitudes(int Lx, int Ly, int D, int chi, const int32_t *dmap, const d
     const int32_t *f = flag ? flag + r0 : nullptr;
     launch_side(g, n, c, f, slots, hdr, st);
     VMCX_LAUNCHED();
-    hipLaunchKernelGGL(peps_bmps_join_kernel, dim3((unsigned)n), dim3(64), 0, st, g, n, c, f,
-                       slots, hdr, 0, 0, sign + r0, logabs + r0, 0, 0, nullptr, nullptr, nullptr,
-                       nullptr);
+    launch_join(g, n, c, f, slots, hdr, 0, 0, sign + r0, logabs + r0, st);
     VMCX_LAUNCHED();
   }
   return 0;
@@ -1534,22 +2264,29 @@ struct BmCacheWs {
   int64_t *chdr, *phdr;
   int32_t *acc;
 };
+// slots for proposals and connected configurations: a launch of one wave per side needs
+// some 8192 configurations to fill the chip (a walker has about as many connected
+// configurations as edges), and its slots are small
+int64_t bm_prop_rows(const BmGeo &g, int64_t B) {
+  if (!bm_wave_fits(g.D, g.cb)) return B;
+  const int64_t p = 8 * B < 8192 ? 8 * B : 8192;
+  return p > B ? p : B;
+}
 BmCacheWs bm_cache_ws(const BmGeo &g, int64_t B, void *ws) {
   BmCacheWs c;
-  const int64_t sd = B * 2 * g.slot;
-  const int64_t hw = B * 2 * g.nbuf * BHDR;
+  const int64_t P = bm_prop_rows(g, B);
   c.cache = (double *)ws;
-  c.prop = c.cache + sd;
-  c.chdr = (int64_t *)(c.prop + sd);
-  c.phdr = c.chdr + hw;
-  c.acc = (int32_t *)(c.phdr + hw);
+  c.prop = c.cache + B * 2 * g.slot;
+  c.chdr = (int64_t *)(c.prop + P * 2 * g.slot);
+  c.phdr = c.chdr + B * 2 * g.nbuf * BHDR;
+  c.acc = (int32_t *)(c.phdr + P * 2 * g.nbuf * BHDR);
   return c;
 }
 }  // namespace
 
 int64_t bmps_sweep_cache_bytes(int Lx, int Ly, int D, int chi, int64_t B) {
   const BmGeo g = bm_cache_geo(Lx, Ly, D, chi);
-  return 2 * B * 2 * g.slot * 8 + 2 * B * 2 * g.nbuf * BHDR * 8 + B * 4;
+  return (B + bm_prop_rows(g, B)) * 2 * (g.slot + g.nbuf * BHDR) * 8 + B * 4;
 }
 
 int32_t *bmps_sweep_accept_flags(int Lx, int Ly, int D, int chi, int64_t B, void *ws) {
@@ -1590,16 +2327,15 @@ int bmps_sweep_amplitudes(int Lx, int Ly, int D, int chi, const int32_t *dmap,
   const int h = Lx / 2;
   launch_side(g, B, pcfg, flag, c.prop, c.phdr, st, st_top, st_bot, c.cache, c.chdr);
   VMCX_LAUNCHED();
-  hipLaunchKernelGGL(peps_bmps_join_kernel, dim3((unsigned)B), dim3(64), 0, st, g, B, pcfg, flag,
-                     c.prop, c.phdr, h - 1, Lx - h - 1, sign, logabs, st_top >= h ? 1 : 0,
-                     st_bot >= Lx - h ? 1 : 0, c.cache, c.chdr, nullptr, nullptr);
+  launch_join(g, B, pcfg, flag, c.prop, c.phdr, h - 1, Lx - h - 1, sign, logabs, st,
+              st_top >= h ? 1 : 0, st_bot >= Lx - h ? 1 : 0, c.cache, c.chdr);
   VMCX_LAUNCHED();
   return 0;
 }
 
 // amplitudes of T connected configurations, each one move (cmove) away from
 // its walker cparent, from the walkers' cached boundaries (bmps_sweep_init
-// of the walkers first), in passes of B through the proposal slots
+// of the walkers first), in passes through the proposal slots
 int bmps_conn_amplitudes(int Lx, int Ly, int D, int chi, const int32_t *dmap,
                          const double *theta, int64_t B, int64_t T, const int64_t *etas,
                          const int32_t *cparent, const uint32_t *cmove, void *ws, double *sign,
@@ -1610,15 +2346,15 @@ int bmps_conn_amplitudes(int Lx, int Ly, int D, int chi, const int32_t *dmap,
   g.theta_stride = 0;
   const BmCacheWs c = bm_cache_ws(g, B, ws);
   const int h = Lx / 2;
-  for (int64_t r0 = 0; r0 < T; r0 += B) {
-    const int64_t n = T - r0 < B ? T - r0 : B;
+  const int64_t P = bm_prop_rows(g, B);
+  for (int64_t r0 = 0; r0 < T; r0 += P) {
+    const int64_t n = T - r0 < P ? T - r0 : P;
     const int64_t *e = etas + r0 * g.N;
     launch_side(g, n, e, nullptr, c.prop, c.phdr, st, 0, 0, c.cache, c.chdr, cparent + r0,
                 cmove + r0);
     VMCX_LAUNCHED();
-    hipLaunchKernelGGL(peps_bmps_join_kernel, dim3((unsigned)n), dim3(64), 0, st, g, n, e,
-                       nullptr, c.prop, c.phdr, h - 1, Lx - h - 1, sign + r0, logabs + r0, 0, 0,
-                       c.cache, c.chdr, cparent + r0, cmove + r0);
+    launch_join(g, n, e, nullptr, c.prop, c.phdr, h - 1, Lx - h - 1, sign + r0, logabs + r0, st,
+                0, 0, c.cache, c.chdr, cparent + r0, cmove + r0);
     VMCX_LAUNCHED();
   }
   return 0;
@@ -1654,9 +2390,7 @@ int bmps_logderiv(int Lx, int Ly, int D, int chi, const int32_t *dmap, const dou
     double *Gr = G + r0 * ldg;
     launch_side(g, n, c, nullptr, slots, hdr, st);
     VMCX_LAUNCHED();
-    hipLaunchKernelGGL(peps_bmps_join_kernel, dim3((unsigned)n), dim3(64), 0, st, g, n, c,
-                       nullptr, slots, hdr, h - 1, Lx - h - 1, sign + r0, logabs + r0, 0, 0,
-                       nullptr, nullptr, nullptr, nullptr);
+    launch_join(g, n, c, nullptr, slots, hdr, h - 1, Lx - h - 1, sign + r0, logabs + r0, st);
     VMCX_LAUNCHED();
     const int64_t nz = n * n_params;
     const unsigned gz = (unsigned)((nz + 255) / 256 < 16384 ? (nz + 255) / 256 : 16384);

@@ -123,6 +123,7 @@ __global__ void __launch_bounds__(256)
 // Builds A^T row-per-lane: a[j] = A[j][col] = M[orb_j][col] + s (D[orb_j*nf+col]
 // + bout[...]) for orb_j the j-th occupied orbital (ascending), with the
 // occupation masks given explicitly (up, dn).
+// (bout NULL: Drow is the compact [nf][nf] of the occupied orbitals, biases added)
 template <int NFP, typename TW>
 __device__ __forceinline__ void nnbf_rows(double (&a)[NFP], uint64_t up, uint64_t dn, int N,
                                           int nf, int col, const TW *__restrict__ M,
@@ -142,7 +143,8 @@ __device__ __forceinline__ void nnbf_rows(double (&a)[NFP], uint64_t up, uint64_
     if (j < nf && col < nf) {
       if (orb >= 0) {
         const int64_t e = (int64_t)orb * nf + col;
-        a[j] = (double)M[e] + s * ((double)Drow[e] + (double)bout[e]);
+        a[j] = (double)M[e] + s * (bout ? (double)Drow[e] + (double)bout[e]
+                                        : (double)Drow[(int64_t)j * nf + col]);
       } else {
         a[j] = 0.0;
       }
@@ -193,7 +195,8 @@ __global__ void __launch_bounds__(256)
   group_masks<NFP>(cfg + w * N, N, col, up, dn);
   const bool count_ok = (__popcll(up) + __popcll(dn)) == nf;
   double a[NFP];
-  nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M, D + w * (int64_t)(2 * N * nf), bout, s);
+  nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M,
+                     D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s);
   const bool nonfinite = group_nonfinite<NFP>(a, grp * NFP);
   const GJResult r = INV ? gj_invert<NFP>(a, col, grp * NFP, prow, qbuf)
                          : lu_logdet<NFP>(a, col, grp * NFP, prow);
@@ -697,6 +700,228 @@ __global__ void __launch_bounds__(256)
   }
 }
 
+// ------------------------------------------------ FP64 dense layers on the matrix cores
+// Occupation masks {up, down} of configuration r (one wave per row); prop given: of the
+// proposed configuration, and none where nothing is proposed
+__device__ __forceinline__ void row_masks(int64_t r, int lane, int N,
+                                          const int64_t *__restrict__ cfg, int i, int j,
+                                          const int32_t *__restrict__ prop, ulonglong2 *masks) {
+  int64_t x = lane < N ? cfg[r * N + lane] : 0;
+  if (prop) {
+    const int p = prop[r];
+    if (lane == i) x = (p >> 8) & 0xF;
+    if (lane == j) x = (p >> 12) & 0xF;
+    if (!(p & 1)) x = 0;
+  }
+  const uint64_t up = __ballot((x & 2) != 0), dn = __ballot((x & 1) != 0);
+  if (lane == 0) masks[r] = make_ulonglong2(up, dn);
+}
+
+struct MaskArgs {
+  const int64_t *cfg;
+  int i, j;
+  const int32_t *prop;
+};
+
+// FP64 layer of a batch with v_mfma_f64_16x16x4f64, rows of h ([R][H]) against blocks of nc
+// rows of the weights ([.][H], the reference's [out][in] layout).
+//   OCC: block o is orbital o's nc = n_f outputs, and only the configurations that occupy o
+//     are taken: A[r][slot of o][c] = acc + bias (compact, [n_f][n_f] per configuration).
+//     The dense product forms every orbital's outputs, the unoccupied half of which no
+//     determinant reads.
+//   otherwise: every row; z (if given) = acc + bias, out = act(acc + bias), [R][H]; further
+//     workgroups write the occupation masks that the OCC product of the batch starts from.
+// A workgroup takes one block and RB configurations: it lists the chosen ones in LDS, its
+// four waves take tiles of 16 RT of them, all nc outputs at once (CT tiles of 16), and share
+// the block's weights through LDS, KC of the sum at a time, loaded one chunk ahead.  A
+// lane's operands of four k-steps are 32 contiguous bytes (the order of the sum over k is
+// free: step kk of lane group g takes k = 16 q + 4 g + kk).  From 8 row blocks on, all
+// workgroups of a row block run on one XCD, whose L2 keeps the rows; spread over all XCDs,
+// each orbital fetched them from beyond L2 (943 us where it takes 737).
+// Bound by the FP64 matrix rate and, at a few thousand rows, by how evenly the orbitals'
+// lists fill tiles and waves.  Measured, 6x6, H = 256, n_f = 32 of 72 orbitals: 54184
+// connected configurations 737 us (dense rocBLAS 1218), 4096 proposals, of which about half
+// are made, 58 us (100); the layer H x H of the former 173 us (190 with bias_act_kernel),
+// of the latter 16 us (18 and 5).
+template <int CT, int RT, int S, bool OCC>
+__global__ void __launch_bounds__(256, 2)
+    nnbf_gemm64_kernel(int64_t R, int RB, int nblk, int ncol, int N, int nc, int H, int act,
+                       const double *__restrict__ W, const double *__restrict__ bias,
+                       const double *__restrict__ h, ulonglong2 *__restrict__ masks,
+                       MaskArgs ma, double *__restrict__ z, double *__restrict__ out) {
+  // NS: weight pairs a thread stages; S: k-steps of rows in flight
+  constexpr int KC = 64, LD = KC + 2, NS = 2 * CT;
+  __shared__ __align__(16) double wl[2][16 * CT * LD];
+  __shared__ int list[OCC ? 1024 : 1];
+  __shared__ int cnt[4];
+  // callers' weights need not be 16-byte aligned
+  typedef double d2 __attribute__((ext_vector_type(2), aligned(8)));
+  typedef double d4 __attribute__((ext_vector_type(4)));
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = lane >> 4;
+  const int64_t nrb = (R + RB - 1) / RB;
+  const bool by_xcd = nrb >= 8;
+  const int64_t slotid = by_xcd ? blockIdx.x >> 3 : blockIdx.x;
+  const int blk = (int)(slotid % nblk), o = blk / ncol, cb = 16 * CT * (blk % ncol);
+  const int64_t r0 = (by_xcd ? (slotid / nblk) * 8 + (blockIdx.x & 7) : slotid / nblk) * RB;
+  if constexpr (!OCC) {
+    const int64_t tiles = (by_xcd ? (nrb + 7) / 8 * 8 : nrb) * nblk, b = blockIdx.x - tiles;
+    if (b >= 0) {
+      for (int64_t r = b * 64 + wave; r < R && r < b * 64 + 64; r += 4)
+        row_masks(r, lane, N, ma.cfg, ma.i, ma.j, ma.prop, masks);
+      return;
+    }
+  }
+  if (r0 >= R) return;
+  const int rb = R - r0 < RB ? (int)(R - r0) : RB;
+  // outputs of the workgroup: ncb from c0 (OCC: from cb of orbital o)
+  const int c0 = o * nc + cb;
+  const int ncb = nc - cb < 16 * CT ? nc - cb : 16 * CT;
+  // staging: pair p = tid + 256 i of a chunk is columns 2 (p % 32), + 1 of row p / 32
+  const double *Ws = W + (int64_t)c0 * H + 2 * (tid & 31);
+  d2 stage[NS];
+  auto fetch = [&](int k) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int c = (tid >> 5) + 8 * i;
+      if (k + 2 * (tid & 31) < H)
+        stage[i] = *reinterpret_cast<const d2 *>(Ws + (int64_t)(c < ncb ? c : ncb - 1) * H + k);
+    }
+  };
+  auto put = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      double *p = &wl[b][((tid >> 5) + 8 * i) * LD + 2 * (tid & 31)];
+      p[0] = stage[i].x;
+      p[1] = stage[i].y;
+    }
+  };
+  fetch(0);
+  int n = 0;
+  if constexpr (OCC) {
+    // local row | slot << 16 of the configurations that occupy o, in row order
+    const int s = o < N ? o : o - N;
+    for (int c0 = 0; c0 < rb; c0 += 256) {
+      const int r = c0 + tid;
+      ulonglong2 m = make_ulonglong2(0, 0);
+      if (r < rb) m = masks[r0 + r];
+      const uint64_t mine = o < N ? m.x : m.y, below = mine & ((1ull << s) - 1);
+      const int slot = __popcll(below) + (o < N ? 0 : __popcll(m.x));
+      // (a configuration with a wrong number of electrons is reported by its determinant:
+      // its surplus orbitals have no slot)
+      const bool on = ((mine >> s) & 1) && slot < nc;
+      const uint64_t b = __ballot(on);
+      if (lane == 0) cnt[wave] = __popcll(b);
+      __syncthreads();
+      int at = n + __popcll(b & ((1ull << lane) - 1));
+      for (int k = 0; k < wave; ++k) at += cnt[k];
+      if (on) list[at] = r | (slot << 16);
+      n += cnt[0] + cnt[1] + cnt[2] + cnt[3];
+      __syncthreads();
+    }
+    if (n == 0) return;
+  } else {
+    n = rb;
+  }
+  const int chunks = (H + KC - 1) / KC;
+  const int groups = (n + 64 * RT - 1) / (64 * RT);
+  int buf = 0;
+  for (int g = 0; g < groups; ++g) {
+    const int t0 = (g * 4 + wave) * 16 * RT;
+    const bool used = t0 < n;
+    const double *hp[RT];
+#pragma unroll
+    for (int t = 0; t < RT; ++t) {
+      const int k = t0 + 16 * t + li, kc = k < n ? k : n - 1;
+      hp[t] = h + (r0 + (OCC ? (list[kc] & 0xFFFF) : kc)) * H + 4 * lk;
+    }
+    d4 acc[RT][CT];
+#pragma unroll
+    for (int a = 0; a < RT; ++a)
+#pragma unroll
+      for (int b = 0; b < CT; ++b) acc[a][b] = (d4){0.0, 0.0, 0.0, 0.0};
+    d2 fa[S][RT][2], ga[S][RT][2];
+    auto load = [&](int k, d2 (&x)[S][RT][2]) {
+#pragma unroll
+      for (int i = 0; i < S; ++i)
+#pragma unroll
+        for (int t = 0; t < RT; ++t)
+#pragma unroll
+          for (int q = 0; q < 2; ++q)
+            x[i][t][q] = reinterpret_cast<const d2 *>(hp[t] + (k + 16 * i < H ? k + 16 * i : 0))[q];
+    };
+    if (used) load(0, fa);
+    for (int ch = 0; ch < chunks; ++ch) {
+      // the buffer was last read two chunks ago, before the barrier of the last one
+      put(buf);
+      __syncthreads();
+      const bool more = ch + 1 < chunks;
+      if (more || g + 1 < groups) fetch(more ? (ch + 1) * KC : 0);
+      if (used) {
+        const double *wb = wl[buf] + li * LD + 4 * lk;
+        auto mult = [&](int k, const d2 (&x)[RT][2]) {
+          d2 y[CT][2];
+#pragma unroll
+          for (int t = 0; t < CT; ++t)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+              y[t][q].x = wb[16 * t * LD + k + 2 * q];
+              y[t][q].y = wb[16 * t * LD + k + 2 * q + 1];
+            }
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int a = 0; a < RT; ++a)
+#pragma unroll
+              for (int b = 0; b < CT; ++b)
+                acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                    q & 1 ? x[a][q >> 1].y : x[a][q >> 1].x,
+                    q & 1 ? y[b][q >> 1].y : y[b][q >> 1].x, acc[a][b], 0, 0, 0);
+        };
+        const int k0 = ch * KC, ke = H - k0 < KC ? H : k0 + KC;
+        for (int k = k0; k < ke; k += 16 * S) {
+          load(k + 16 * S, ga);
+          __builtin_amdgcn_sched_barrier(0);   // (the loads would sink to their use)
+#pragma unroll
+          for (int i = 0; i < S; ++i)
+            if (i == 0 || k + 16 * i < ke) mult(k + 16 * i - k0, fa[i]);
+          __builtin_amdgcn_sched_barrier(0);   // (nor are they waited for before)
+#pragma unroll
+          for (int i = 0; i < S; ++i)
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+              fa[i][t][0] = ga[i][t][0];
+              fa[i][t][1] = ga[i][t][1];
+            }
+        }
+      }
+      buf ^= 1;
+    }
+    // result register r of lane l: row 4 r + l / 16 of the tile, output l % 16
+#pragma unroll
+    for (int b = 0; b < CT; ++b) {
+      const int c = 16 * b + li;
+      if (c >= ncb) continue;
+      const double bv = bias[c0 + c];
+#pragma unroll
+      for (int a = 0; a < RT; ++a)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int k = t0 + 16 * a + 4 * r + lk;
+          if (k >= n) continue;
+          const double v = acc[a][b][r] + bv;
+          if constexpr (OCC) {
+            const int e = list[k];
+            out[((r0 + (e & 0xFFFF)) * nc + (e >> 16)) * nc + cb + c] = v;
+          } else {
+            const int64_t e = (r0 + k) * H + c0 + c;
+            if (z) z[e] = v;
+            out[e] = act_f(v, act);
+          }
+        }
+    }
+  }
+}
+
 // ------------------------------------------------------------ sweep pieces
 // prop[w] = flag | ni << 8 | nj << 12 | nmoves << 16 ; moves[w] = a1 b1 a2 b2 (bytes)
 __global__ void __launch_bounds__(256)
@@ -893,7 +1118,8 @@ __global__ void __launch_bounds__(256)
   dn = (dn & ~((1ull << i) | (1ull << j))) | ((uint64_t)(ni & 1) << i) |
        ((uint64_t)(nj & 1) << j);
   double a[NFP];
-  nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M, D + w * (int64_t)(2 * N * nf), bout, s);
+  nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M,
+                     D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s);
   const GJResult r = lu_logdet<NFP>(a, col, grp * NFP, prow);
   const double lp = r.singular ? log(1e-45) : fmax(r.logdet, log(1e-45));
   const double ratio = exp(2.0 * (lp - logabs[w]));
@@ -1209,6 +1435,7 @@ struct NnbfWs {
   int32_t *prop;
   uint32_t *moves;
   double *uacc;
+  ulonglong2 *masks;   // FP64: occupations of the batch's rows
   // local-energy buffers
   int64_t *counts, *offsets, *total, *etas;
   double *coeffs, *csign, *clog;
@@ -1240,6 +1467,7 @@ static NnbfWs nnbf_layout(const vmcx_nnbf_model &m, int64_t B, int64_t chunk, in
   L.h2 = take((size_t)chunk * H * ti);
   L.g1 = take((size_t)chunk * H * tw);
   L.g2 = take((size_t)chunk * H * tw);
+  L.masks = (ulonglong2 *)L.g2;   // (H >= 16 there; g2 is the backward's)
   L.ainv = (double *)take((size_t)chunk * nfp * nfp * 8);
   L.prop = (int32_t *)take((size_t)B * 4);
   L.moves = (uint32_t *)take((size_t)B * 4);
@@ -1314,6 +1542,67 @@ static int nn_gemm(rocblas_handle h, rocblas_operation ta, int mm, int nn, int k
 }
 
 // z2 = W2 h1 ; D = Wout act(z2 + b2)  for `rows` rows already holding h1
+// FP64 layers by nnbf_gemm64_kernel: whole 16-wide k-steps, and the occupied orbitals'
+// outputs, padded to tiles of 16, at most 0.6 of the dense product that rocBLAS forms.
+// Measured (whole sampling pass, dense -> occupied): at 0.5 gains of 4 to 12 % (4x4 half
+// filled, n_f 12 and 16, 300 to 4096 configurations), 0.44 (6x6, n_f = 32) 25 %; at 0.67
+// (6x6, n_f = 36) losses of 3 to 6 % at 300 to 1000 and a gain of 2 % at 4096.
+static bool occ64(const vmcx_nnbf_model &m) {
+  return m.gemm == 2 && m.hidden % 16 == 0 && (m.n_f + 15) / 16 * 16 * 5 <= 3 * 2 * m.n_sites;
+}
+
+template <int CT, int RT, int S, bool OCC>
+static void launch_gemm64(int64_t R, int RB, int groups, int N, int nc, int H, int act,
+                          const double *W, const double *bias, const double *h,
+                          ulonglong2 *masks, const MaskArgs &ma, double *z, double *out,
+                          hipStream_t st) {
+  const int ncol = (nc + 16 * CT - 1) / (16 * CT);
+  int64_t rblocks = (R + RB - 1) / RB;
+  if (rblocks >= 8) rblocks = (rblocks + 7) / 8 * 8;
+  const int64_t grid = rblocks * groups * ncol + (OCC ? 0 : (R + 63) / 64);
+  hipLaunchKernelGGL((nnbf_gemm64_kernel<CT, RT, S, OCC>), dim3((unsigned)grid), dim3(256), 0, st,
+                     R, RB, groups * ncol, ncol, N, nc, H, act, W, bias, h, masks, ma, z, out);
+}
+
+// layer 2 and the occupied orbitals' outputs (L.D compact); prop: of the proposals of edge
+// (i, j).  keep_z: the pre-activations z2 for the backward
+template <int CT2, int RT2, int S2, int CT, int RT, int S>
+static int dense_layers64(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t rows, int RB2,
+                          int RB, const MaskArgs &ma, bool keep_z, hipStream_t st) {
+  const NnW<double> W = weights_of<double>(m);
+  const int H = m.hidden, N = m.n_sites;
+  double *h2 = (double *)L.h2;
+  launch_gemm64<CT2, RT2, S2, false>(rows, RB2, 1, N, H, H, m.act, W.W2, W.b2,
+                                     (const double *)L.h1, L.masks, ma,
+                                     keep_z ? (double *)L.z2 : nullptr, h2, st);
+  launch_gemm64<CT, RT, S, true>(rows, RB, 2 * N, N, m.n_f, H, 0, W.Wout, W.bout, h2, L.masks, ma,
+                                 nullptr, (double *)L.D, st);
+  VMCX_LAUNCHED();
+  return 0;
+}
+
+static int dense_layers64(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t rows,
+                          const int64_t *cfg, int i, int j, const int32_t *prop, bool keep_z,
+                          hipStream_t st) {
+  const MaskArgs ma = {cfg, i, j, prop};
+  const int ct = m.n_f <= 16 ? 1 : m.n_f > 32 && m.n_f <= 48 ? 3 : 2;   // least padding
+  if (rows <= 1024) {
+    // latency: narrow tiles of layer 2, four k-steps of rows in flight
+    if (ct == 1) return dense_layers64<1, 1, 4, 1, 1, 4>(m, L, rows, 64, 128, ma, keep_z, st);
+    if (ct == 2) return dense_layers64<1, 1, 4, 2, 1, 4>(m, L, rows, 64, 128, ma, keep_z, st);
+    return dense_layers64<1, 1, 4, 3, 1, 4>(m, L, rows, 64, 128, ma, keep_z, st);
+  }
+  if (rows <= 16384) {
+    // enough tiles of 16 rows for the chip's waves
+    if (ct == 1) return dense_layers64<2, 1, 1, 1, 1, 1>(m, L, rows, 64, 256, ma, keep_z, st);
+    if (ct == 2) return dense_layers64<2, 1, 1, 2, 1, 1>(m, L, rows, 64, 256, ma, keep_z, st);
+    return dense_layers64<2, 1, 1, 3, 1, 1>(m, L, rows, 64, 256, ma, keep_z, st);
+  }
+  if (ct == 1) return dense_layers64<2, 2, 1, 1, 2, 1>(m, L, rows, 256, 1024, ma, keep_z, st);
+  if (ct == 2) return dense_layers64<2, 2, 1, 2, 2, 1>(m, L, rows, 256, 1024, ma, keep_z, st);
+  return dense_layers64<2, 2, 1, 3, 2, 1>(m, L, rows, 256, 1024, ma, keep_z, st);
+}
+
 template <typename TW, typename TI>
 static int dense_layers(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t rows,
                         hipStream_t st) {
@@ -1343,14 +1632,15 @@ static void launch_det(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t rows,
   const int64_t per_block = 4 * WPW;
   const int64_t nblk = (rows + per_block - 1) / per_block;
   const NnW<TW> W = weights_of<TW>(m);
+  const TW *bout = occ64(m) ? nullptr : W.bout;
   if (ainv)
     hipLaunchKernelGGL((nnbf_det_kernel<NFP, true, TW>), dim3((unsigned)nblk), dim3(256),
                        (size_t)per_block * NFP * 9, st, rows, m.n_sites, m.n_f, cfg,
-                       (const TW *)L.D, W.M, W.bout, m.bf_scale, sign, logabs, ainv);
+                       (const TW *)L.D, W.M, bout, m.bf_scale, sign, logabs, ainv);
   else
     hipLaunchKernelGGL((nnbf_det_kernel<NFP, false, TW>), dim3((unsigned)nblk), dim3(256),
                        (size_t)per_block * NFP * 9, st, rows, m.n_sites, m.n_f, cfg,
-                       (const TW *)L.D, W.M, W.bout, m.bf_scale, sign, logabs, ainv);
+                       (const TW *)L.D, W.M, bout, m.bf_scale, sign, logabs, ainv);
 }
 
 template <typename TW, typename TI>
@@ -1478,7 +1768,8 @@ static int forward_rows_t(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t row
   if (rows == 0) return 0;
   int rc = h1_ready ? 0 : layer1<TW, TI>(m, L, rows, cfg, st);
   if (rc) return rc;
-  rc = dense_layers<TW, TI>(m, L, rows, st);
+  rc = occ64(m) ? dense_layers64(m, L, rows, cfg, 0, 0, nullptr, ainv != nullptr, st)
+                : dense_layers<TW, TI>(m, L, rows, st);
   if (rc) return rc;
   switch (nfp_of(m.n_f)) {
     case 8: launch_det<8, TW>(m, L, rows, cfg, sign, logabs, ainv, st); break;
@@ -1633,8 +1924,8 @@ static void launch_accept(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t B, 
   const NnW<TW> W = weights_of<TW>(m);
   hipLaunchKernelGGL((nnbf_accept_kernel<NFP, TW>), dim3((unsigned)nblk), dim3(256),
                      (size_t)per_block * NFP * 9, st, B, m.n_sites, m.n_f, m.hidden, i, j, cfg,
-                     L.prop, L.moves, L.uacc, (const TW *)L.D, W.M, W.bout, m.bf_scale, W.W1,
-                     z1, sign, logabs, n_accept);
+                     L.prop, L.moves, L.uacc, (const TW *)L.D, W.M,
+                     occ64(m) ? nullptr : W.bout, m.bf_scale, W.W1, z1, sign, logabs, n_accept);
 }
 
 template <typename TW, typename TI>
@@ -1647,7 +1938,8 @@ static int sweep_edge(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t B, int 
   hipLaunchKernelGGL((nnbf_h1_proposed_kernel<TW, TI>), dim3(gh), dim3(256), 0, st, B,
                      m.n_sites, m.hidden, m.act, W.W1, z1, L.prop, L.moves, (TI *)L.h1);
   VMCX_LAUNCHED();
-  const int rc = dense_layers<TW, TI>(m, L, B, st);
+  const int rc = occ64(m) ? dense_layers64(m, L, B, cfg, i, j, L.prop, false, st)
+                          : dense_layers<TW, TI>(m, L, B, st);
   if (rc) return rc;
   switch (nfp_of(m.n_f)) {
     case 8: launch_accept<8, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, st); break;

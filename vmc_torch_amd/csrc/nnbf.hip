@@ -924,39 +924,46 @@ __global__ void __launch_bounds__(256, 2)
 
 // ------------------------------------------------------------ sweep pieces
 // prop[w] = flag | ni << 8 | nj << 12 | nmoves << 16 ; moves[w] = a1 b1 a2 b2 (bytes)
-__global__ void __launch_bounds__(256)
-    nnbf_propose_kernel(int64_t B, int N, int i, int j, int e, int64_t sweep,
-                        uint64_t seed, double keep_rate, const double *u_choice,
-                        const uint8_t *bits, const double *u_acc_in,
-                        const int64_t *__restrict__ cfg, int32_t *prop, uint32_t *moves,
-                        double *u_acc) {
-  const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= B) return;
-  const int si = (int)cfg[w * N + i], sj = (int)cfg[w * N + j];
+// draws of one edge: Philox, or injected ([B] each)
+struct ProposeArgs {
+  int i, j, e;
+  int64_t sweep;
+  uint64_t seed;
+  double keep_rate;
+  const double *u_choice, *u_acc_in;
+  const uint8_t *bits;
+  int32_t *prop;
+  uint32_t *moves;
+  double *u_acc;
+};
+
+__device__ __forceinline__ void propose_one(int64_t w, int N, const ProposeArgs &A, int si,
+                                            int sj) {
+  const int i = A.i, j = A.j;
   if (si == sj) {
-    prop[w] = 0;
+    A.prop[w] = 0;
     return;
   }
   double uc, ua;
   int b0, b2;
-  if (u_choice == nullptr) {
-    const u32x4 o = philox4x32_10((uint32_t)e, (uint32_t)sweep, (uint32_t)w, 0u,
-                                  (uint32_t)seed, (uint32_t)(seed >> 32));
+  if (A.u_choice == nullptr) {
+    const u32x4 o = philox4x32_10((uint32_t)A.e, (uint32_t)A.sweep, (uint32_t)w, 0u,
+                                  (uint32_t)A.seed, (uint32_t)(A.seed >> 32));
     uc = u53(o.x, o.y);
     ua = u53(o.z, o.w);
     b0 = o.y & 1u;
     b2 = (o.y >> 1) & 1u;
   } else {
-    uc = u_choice[w];
-    ua = u_acc_in[w];
-    b0 = bits[w] & 1;
-    b2 = (bits[w] >> 1) & 1;
+    uc = A.u_choice[w];
+    ua = A.u_acc_in[w];
+    b0 = A.bits[w] & 1;
+    b2 = (A.bits[w] >> 1) & 1;
   }
   const int nmi = (si == 0) ? 0 : ((si == 3) ? 2 : 1);
   const int nmj = (sj == 0) ? 0 : ((sj == 3) ? 2 : 1);
   const int dnum = nmi > nmj ? nmi - nmj : nmj - nmi;
   int ni, nj;
-  if (uc < keep_rate || dnum == 1) {
+  if (uc < A.keep_rate || dnum == 1) {
     ni = sj;
     nj = si;
   } else if (dnum == 0) {
@@ -978,19 +985,30 @@ __global__ void __launch_bounds__(256)
     mv |= (uint32_t)((N + from) | ((N + to) << 8)) << (16 * nm);
     ++nm;
   }
-  prop[w] = 1 | (ni << 8) | (nj << 12) | (nm << 16);
-  moves[w] = mv;
-  u_acc[w] = ua;
+  A.prop[w] = 1 | (ni << 8) | (nj << 12) | (nm << 16);
+  A.moves[w] = mv;
+  A.u_acc[w] = ua;
+}
+
+__global__ void __launch_bounds__(256)
+    nnbf_propose_kernel(int64_t B, int N, int i, int j, int e, int64_t sweep,
+                        uint64_t seed, double keep_rate, const double *u_choice,
+                        const uint8_t *bits, const double *u_acc_in,
+                        const int64_t *__restrict__ cfg, int32_t *prop, uint32_t *moves,
+                        double *u_acc) {
+  const int64_t w = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (w >= B) return;
+  propose_one(w, N, {i, j, e, sweep, seed, keep_rate, u_choice, u_acc_in, bits, prop, moves, u_acc},
+              (int)cfg[w * N + i], (int)cfg[w * N + j]);
 }
 
 // h1p = act(z1 + sum_moves (W1[:, to] - W1[:, from]))
 template <typename TW, typename TI>
 __global__ void __launch_bounds__(256)
-    nnbf_h1_proposed_kernel(int64_t B, int N, int H, int act, const TW *__restrict__ W1,
+    nnbf_h1_proposed_kernel(int64_t B, int H, int act, const TW *__restrict__ W1T,
                             const TW *__restrict__ z1, const int32_t *__restrict__ prop,
                             const uint32_t *__restrict__ moves, TI *h1p) {
   const int64_t n = B * H;
-  const int n_orb = 2 * N;
   for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < n;
        idx += (int64_t)gridDim.x * blockDim.x) {
     const int64_t w = idx / H;
@@ -1002,7 +1020,7 @@ __global__ void __launch_bounds__(256)
       const uint32_t mv = moves[w];
       for (int m = 0; m < nm; ++m) {
         const int from = (mv >> (16 * m)) & 0xFF, to = (mv >> (16 * m + 8)) & 0xFF;
-        z += W1[(int64_t)u * n_orb + to] - W1[(int64_t)u * n_orb + from];
+        z += W1T[(int64_t)to * H + u] - W1T[(int64_t)from * H + u];
       }
     }
     h1p[idx] = to_t<TI>(act_f(z, act));
@@ -1089,15 +1107,17 @@ __global__ void masked_rows_kernel(int64_t B, int64_t row_words, const uint8_t *
     if (mask[idx / row_words]) dst[idx] = src[idx];
 }
 
-// determinant of the proposed configuration, Metropolis test, commit
+// Determinant of the proposed configuration, Metropolis test, commit; then the walker's
+// proposal on the next edge (if `more`).  The commit's columns of W1 are read from the
+// transposed weights, eight of a lane's units in flight (read by rows of W1, one unit at a
+// time, they were a third of the kernel's latency; TACC).
 template <int NFP, typename TW>
 __global__ void __launch_bounds__(256)
     nnbf_accept_kernel(int64_t B, int N, int nf, int H, int i, int j, int64_t *cfg,
-                       const int32_t *__restrict__ prop, const uint32_t *__restrict__ moves,
-                       const double *__restrict__ u_acc, const TW *__restrict__ D,
-                       const TW *__restrict__ M, const TW *__restrict__ bout, double s,
-                       const TW *__restrict__ W1, TW *z1, double *sign, double *logabs,
-                       int64_t *n_accept) {
+                       const TW *__restrict__ D, const TW *__restrict__ M,
+                       const TW *__restrict__ bout, double s, const TW *__restrict__ W1T,
+                       TW *z1, double *sign, double *logabs, int64_t *n_accept,
+                       ProposeArgs next, bool more) {
   constexpr int WPW = 64 / NFP;
   extern __shared__ __align__(16) char smem[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1106,43 +1126,55 @@ __global__ void __launch_bounds__(256)
   const int per_block = (blockDim.x / 64) * WPW;
   const int64_t w = (int64_t)blockIdx.x * per_block + wl;
   if (w >= B) return;
-  const int p = prop[w];
-  if (!(p & 1)) return;
-  double *prow = reinterpret_cast<double *>(smem) + wl * NFP;
-  const int ni = (p >> 8) & 0xF, nj = (p >> 12) & 0xF;
-  uint64_t up, dn;
-  group_masks<NFP>(cfg + w * N, N, col, up, dn);
-  // proposed occupation
-  up = (up & ~((1ull << i) | (1ull << j))) | ((uint64_t)((ni >> 1) & 1) << i) |
-       ((uint64_t)((nj >> 1) & 1) << j);
-  dn = (dn & ~((1ull << i) | (1ull << j))) | ((uint64_t)(ni & 1) << i) |
-       ((uint64_t)(nj & 1) << j);
-  double a[NFP];
-  nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M,
-                     D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s);
-  const GJResult r = lu_logdet<NFP>(a, col, grp * NFP, prow);
-  const double lp = r.singular ? log(1e-45) : fmax(r.logdet, log(1e-45));
-  const double ratio = exp(2.0 * (lp - logabs[w]));
-  if (!(u_acc[w] < ratio)) return;
-  // commit (group-uniform branch)
-  if (col == 0) {
-    cfg[w * N + i] = ni;
-    cfg[w * N + j] = nj;
-    sign[w] = r.singular ? 0.0 : ((r.parity & 1) ? -1.0 : 1.0);
-    logabs[w] = lp;
-    if (n_accept) n_accept[w] += 1;
-  }
-  const int nm = (p >> 16) & 3;
-  const uint32_t mv = moves[w];
-  const int n_orb = 2 * N;
-  for (int u = col; u < H; u += NFP) {
-    TW dz = 0;
-    for (int m = 0; m < nm; ++m) {
-      const int from = (mv >> (16 * m)) & 0xFF, to = (mv >> (16 * m + 8)) & 0xFF;
-      dz += W1[(int64_t)u * n_orb + to] - W1[(int64_t)u * n_orb + from];
+  const int p = next.prop[w];
+  if (p & 1) {
+    double *prow = reinterpret_cast<double *>(smem) + wl * NFP;
+    const int ni = (p >> 8) & 0xF, nj = (p >> 12) & 0xF;
+    uint64_t up, dn;
+    group_masks<NFP>(cfg + w * N, N, col, up, dn);
+    // proposed occupation
+    up = (up & ~((1ull << i) | (1ull << j))) | ((uint64_t)((ni >> 1) & 1) << i) |
+         ((uint64_t)((nj >> 1) & 1) << j);
+    dn = (dn & ~((1ull << i) | (1ull << j))) | ((uint64_t)(ni & 1) << i) |
+         ((uint64_t)(nj & 1) << j);
+    double a[NFP];
+    nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M,
+                       D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s);
+    const GJResult r = lu_logdet<NFP>(a, col, grp * NFP, prow);
+    const double lp = r.singular ? log(1e-45) : fmax(r.logdet, log(1e-45));
+    const double ratio = exp(2.0 * (lp - logabs[w]));
+    if (next.u_acc[w] < ratio) {   // (group-uniform branch)
+      if (col == 0) {
+        cfg[w * N + i] = ni;
+        cfg[w * N + j] = nj;
+        sign[w] = r.singular ? 0.0 : ((r.parity & 1) ? -1.0 : 1.0);
+        logabs[w] = lp;
+        if (n_accept) n_accept[w] += 1;
+      }
+      const int nm = (p >> 16) & 3;
+      const uint32_t mv = next.moves[w];
+      const TW *f0 = W1T + (int64_t)(mv & 0xFF) * H, *t0 = W1T + (int64_t)((mv >> 8) & 0xFF) * H;
+      const TW *f1 = W1T + (int64_t)((mv >> 16) & 0xFF) * H, *t1 = W1T + (int64_t)(mv >> 24) * H;
+      TW *zw = z1 + w * H;
+      for (int u0 = col; u0 < H; u0 += 8 * NFP) {
+        TW dz[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int u = u0 + k * NFP;
+          dz[k] = 0;
+          if (u < H && nm > 0) dz[k] += t0[u] - f0[u];
+          if (u < H && nm > 1) dz[k] += t1[u] - f1[u];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const int u = u0 + k * NFP;
+          if (u < H) zw[u] += dz[k];
+        }
+      }
     }
-    z1[w * H + u] += dz;
   }
+  if (more && col == 0)
+    propose_one(w, N, next, (int)cfg[w * N + next.i], (int)cfg[w * N + next.j]);
 }
 
 // ------------------------------------------------------------ local energy
@@ -1917,35 +1949,35 @@ int nnbf_forward(const vmcx_nnbf_model *m, int64_t B, const int64_t *cfg, void *
 template <int NFP, typename TW>
 static void launch_accept(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t B, int i, int j,
                           int64_t *cfg, TW *z1, double *sign, double *logabs,
-                          int64_t *n_accept, hipStream_t st) {
+                          int64_t *n_accept, const ProposeArgs &next, bool more,
+                          hipStream_t st) {
   constexpr int WPW = 64 / NFP;
   const int64_t per_block = 4 * WPW;
   const int64_t nblk = (B + per_block - 1) / per_block;
   const NnW<TW> W = weights_of<TW>(m);
   hipLaunchKernelGGL((nnbf_accept_kernel<NFP, TW>), dim3((unsigned)nblk), dim3(256),
                      (size_t)per_block * NFP * 9, st, B, m.n_sites, m.n_f, m.hidden, i, j, cfg,
-                     L.prop, L.moves, L.uacc, (const TW *)L.D, W.M,
-                     occ64(m) ? nullptr : W.bout, m.bf_scale, W.W1, z1, sign, logabs, n_accept);
+                     (const TW *)L.D, W.M, occ64(m) ? nullptr : W.bout, m.bf_scale,
+                     (const TW *)L.w1t, z1, sign, logabs, n_accept, next, more);
 }
 
 template <typename TW, typename TI>
 static int sweep_edge(const vmcx_nnbf_model &m, const NnbfWs &L, int64_t B, int i, int j,
                       int64_t *cfg, TW *z1, double *sign, double *logabs, int64_t *n_accept,
-                      hipStream_t st) {
+                      const ProposeArgs &next, bool more, hipStream_t st) {
   const int64_t nh = B * m.hidden;
   const unsigned gh = (unsigned)((nh + 255) / 256 < 16384 ? (nh + 255) / 256 : 16384);
-  const NnW<TW> W = weights_of<TW>(m);
   hipLaunchKernelGGL((nnbf_h1_proposed_kernel<TW, TI>), dim3(gh), dim3(256), 0, st, B,
-                     m.n_sites, m.hidden, m.act, W.W1, z1, L.prop, L.moves, (TI *)L.h1);
+                     m.hidden, m.act, (const TW *)L.w1t, z1, L.prop, L.moves, (TI *)L.h1);
   VMCX_LAUNCHED();
   const int rc = occ64(m) ? dense_layers64(m, L, B, cfg, i, j, L.prop, false, st)
                           : dense_layers<TW, TI>(m, L, B, st);
   if (rc) return rc;
   switch (nfp_of(m.n_f)) {
-    case 8: launch_accept<8, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, st); break;
-    case 16: launch_accept<16, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, st); break;
-    case 32: launch_accept<32, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, st); break;
-    default: launch_accept<64, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, st); break;
+    case 8: launch_accept<8, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, next, more, st); break;
+    case 16: launch_accept<16, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, next, more, st); break;
+    case 32: launch_accept<32, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, next, more, st); break;
+    default: launch_accept<64, TW>(m, L, B, i, j, cfg, z1, sign, logabs, n_accept, next, more, st); break;
   }
   VMCX_LAUNCHED();
   return 0;
@@ -1971,28 +2003,44 @@ int nnbf_sweep(const vmcx_nnbf_model *m, int64_t B, int n_edges, const int32_t *
     const int i = edges_host[2 * e], j = edges_host[2 * e + 1];
     VMCX_CHECK_ARG(i >= 0 && i < N && j >= 0 && j < N && i != j, "edge out of range");
   }
-  const unsigned gw = (unsigned)((B + 255) / 256);
-  for (int sw = 0; sw < n_sweeps; ++sw) {
-    for (int e = 0; e < n_edges; ++e) {
-      const int i = edges_host[2 * e], j = edges_host[2 * e + 1];
-      const size_t di = ((size_t)sw * n_edges + e) * B;
-      hipLaunchKernelGGL(nnbf_propose_kernel, dim3(gw), dim3(256), 0, st, B, N, i, j, e,
-                         sweep_offset + sw, seed, 1.0 - hopping_rate,
-                         u_choice ? u_choice + di : nullptr, bits ? bits + di : nullptr,
-                         u_acc ? u_acc + di : nullptr, cfg, L.prop, L.moves, L.uacc);
-      VMCX_LAUNCHED();
-      int rc;
-      if (m->gemm == 2)
-        rc = sweep_edge<double, double>(*m, L, B, i, j, cfg, (double *)z1, sign, logabs,
-                                        n_accept, st);
-      else if (m->gemm == 1)
-        rc = sweep_edge<float, __hip_bfloat16>(*m, L, B, i, j, cfg, (float *)z1, sign, logabs,
-                                               n_accept, st);
-      else
-        rc = sweep_edge<float, float>(*m, L, B, i, j, cfg, (float *)z1, sign, logabs, n_accept,
-                                      st);
-      if (rc) return rc;
-    }
+  if (n_sweeps == 0 || n_edges == 0) return 0;
+  const int64_t steps = (int64_t)n_sweeps * n_edges, nw = (int64_t)m->hidden * 2 * N;
+  auto args = [&](int64_t k) {
+    const int e = (int)(k % n_edges);
+    const size_t d = (size_t)k * B;
+    return ProposeArgs{edges_host[2 * e], edges_host[2 * e + 1], e, sweep_offset + k / n_edges,
+                       seed, 1.0 - hopping_rate, u_choice ? u_choice + d : nullptr,
+                       u_acc ? u_acc + d : nullptr, bits ? bits + d : nullptr, L.prop, L.moves,
+                       L.uacc};
+  };
+  const dim3 gw((unsigned)((B + 255) / 256)), gt((unsigned)((nw + 255) / 256));
+  if (m->gemm == 2)
+    hipLaunchKernelGGL((nnbf_w1t_kernel<double>), gt, dim3(256), 0, st, m->hidden, 2 * N,
+                       weights_of<double>(*m).W1, (double *)L.w1t);
+  else
+    hipLaunchKernelGGL((nnbf_w1t_kernel<float>), gt, dim3(256), 0, st, m->hidden, 2 * N,
+                       weights_of<float>(*m).W1, (float *)L.w1t);
+  const ProposeArgs A = args(0);
+  hipLaunchKernelGGL(nnbf_propose_kernel, gw, dim3(256), 0, st, B, N, A.i, A.j, A.e, A.sweep,
+                     A.seed, A.keep_rate, A.u_choice, A.bits, A.u_acc_in, cfg, A.prop, A.moves,
+                     A.u_acc);
+  VMCX_LAUNCHED();
+  for (int64_t k = 0; k < steps; ++k) {
+    const ProposeArgs cur = args(k);
+    const bool more = k + 1 < steps;
+    const ProposeArgs next = more ? args(k + 1) : cur;
+    const int i = cur.i, j = cur.j;
+    int rc;
+    if (m->gemm == 2)
+      rc = sweep_edge<double, double>(*m, L, B, i, j, cfg, (double *)z1, sign, logabs, n_accept,
+                                      next, more, st);
+    else if (m->gemm == 1)
+      rc = sweep_edge<float, __hip_bfloat16>(*m, L, B, i, j, cfg, (float *)z1, sign, logabs,
+                                             n_accept, next, more, st);
+    else
+      rc = sweep_edge<float, float>(*m, L, B, i, j, cfg, (float *)z1, sign, logabs, n_accept,
+                                    next, more, st);
+    if (rc) return rc;
   }
   return 0;
 }

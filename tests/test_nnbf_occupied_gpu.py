@@ -58,3 +58,37 @@ def test_occupied_outputs_wrong_count(device):
     keep = [r for r in range(40) if r not in (3, 17)]
     assert torch.isnan(l[[3, 17]]).all()
     assert torch.equal(s[keep], good[0][keep]) and torch.equal(l[keep], good[1][keep])
+
+
+# the 64-lane elimination: one column in the last panel, full panels, one more
+@pytest.mark.parametrize("nu,nd", [(17, 16), (24, 24), (25, 24), (32, 32)])
+def test_determinant_panels(device, nu, nd):
+    """Entries that leave no choice of pivot (one nonzero per row and column, in random
+    order), so that sign and magnitude are exact up to the logarithms' rounding, 1e-12 of a
+    sum of at most 64; the same with an empty column is singular."""
+    rng = np.random.default_rng(nu)
+    nf, N = nu + nd, 64
+    x = np.zeros((6, N), np.int64)
+    M = np.zeros((2 * N, nf))
+    sites_up, sites_dn = rng.permutation(N)[:nu], rng.permutation(N)[:nd]
+    x[:, sites_up] += 2
+    x[:, sites_dn] += 1
+    orb = np.concatenate([np.sort(sites_up), N + np.sort(sites_dn)])
+    perm = rng.permutation(nf)
+    M[orb, perm] = rng.choice([-1.0, 1.0], nf) * np.exp2(rng.integers(-3, 4, nf))
+    A = M[orb]
+    for empty in (None, 0, nf - 1):
+        Me = M.copy()
+        if empty is not None:
+            Me[:, empty] = 0
+        for gemm in ("fp64", "bf16"):
+            m = NNBF_GPU(N, nf, hidden_dim=32, bf_scale=0.0, gemm=gemm, init="xavier").to(device)
+            with torch.no_grad():
+                [p for p in m.params if tuple(p.shape) == Me.shape][0].copy_(torch.tensor(Me))
+            s, l = m.forward_log(torch.tensor(x, device=device))
+            if empty is None:
+                so, lo = np.linalg.slogdet(A)
+                assert (s.cpu().numpy() == so).all()
+                assert np.abs(l.cpu().numpy() - lo).max() < 1e-12 * max(1.0, 64 * np.log(8.0))
+            else:
+                assert (s == 0).all() and (l.cpu().numpy() == np.log(1e-45)).all()

@@ -246,22 +246,20 @@ struct LuStep<NFP, NFP, T> {
   static __device__ __forceinline__ void run(T (&)[NFP], int, int, T *, LuState &) {}
 };
 
-// One 64 x 64 matrix per wave: the pivot is the same for every lane, so the
-// arg-max is a DPP max-scan (row_shr 1, 2, 4, 8, row_bcast 15, 31; the wave
-// maximum ends in lane 63).  The pivot row reaches the other lanes two ways
-// at once: its head by readlane into scalar registers (two VALU
-// instructions per entry with the update), its tail through the wave's
-// 64-entry LDS buffer (written by the pivot lane as 16-byte vectors, read
-// back by every lane as broadcasts: one VALU instruction per entry); the
-// tail takes 4/6 of the entries in FP32, 3/6 in FP64, the split that keeps
-// both the VALU and the LDS pipes busy.  Every lane applies the update, the
-// pivot lane with multiplier exactly 1: its registers past P become exact
-// zeros, so a lane once chosen keys at most 63 (the lane bits alone) at
-// every later step and loses to any unchosen lane with a nonzero entry; no
-// per-lane "done" test is needed.  (If every unchosen entry is zero the
-// matrix is singular and whichever lane wins carries a zero pivot.)  The
-// pivot of each step is kept in the chosen lane of `pivs`; sign and
-// log|det| are formed from them once, after the last step (lu64_finish).
+// One 64 x 64 matrix per wave, in four panels of 16 columns: the panel is eliminated with a
+// row per lane, the columns right of it take the panel's update on the matrix cores, in
+// between in the matrix-core result layout.  Every lane applies every step, the pivot lane
+// with multiplier exactly 1: its row becomes exact zeros, so a lane once chosen keys at most
+// 63 (the lane bits alone) at every later step and loses to any unchosen lane with a nonzero
+// entry; no per-lane "done" test is needed.  (If every unchosen entry is zero the matrix is
+// singular and whichever lane wins carries a zero pivot.)  The pivot of each step is kept in
+// the chosen lane of `pivs`; sign and log|det| are formed from them once, after the last
+// step (lu64_finish).
+// Bound by the vector instructions and the dependent chain of the 64 pivot searches.  A
+// step of the unblocked elimination updates up to 63 entries of a lane with up to 63
+// broadcasts, and its 64 unrolled steps exceed the instruction cache; here it is 15 and 15,
+// and the four panels share one code.  Measured, with the loads of nnbf_detA_kernel: 65536
+// FP32 determinants 707 -> 502 us; one wave's FP64 determinant in nnbf_accept_kernel 64 -> 38 us.
 // multiplier a / piv: FP32 by the hardware reciprocal (1 ulp), FP64 by the
 // correctly rounded division
 __device__ __forceinline__ float lu_mult(float a, float piv) {
@@ -275,7 +273,7 @@ struct LuVec;
 template <>
 struct LuVec<float> {
   typedef float4 t;
-  static constexpr int n = 4, tail6 = 4;
+  static constexpr int n = 4;
   static __device__ __forceinline__ t make(const float *x) {
     return make_float4(x[0], x[1], x[2], x[3]);
   }
@@ -283,77 +281,216 @@ struct LuVec<float> {
 template <>
 struct LuVec<double> {
   typedef double2 t;
-  static constexpr int n = 2, tail6 = 3;
+  static constexpr int n = 2;
   static __device__ __forceinline__ t make(const double *x) { return make_double2(x[0], x[1]); }
 };
+// Exchange of register blocks and lane groups: reg[c] of lane group g <-> reg[g] of lane
+// group c (groups of 16 lanes, four registers).
+__device__ __forceinline__ void lu_swap4(uint32_t &r0, uint32_t &r1, uint32_t &r2, uint32_t &r3) {
+  auto x = __builtin_amdgcn_permlane32_swap(r0, r2, false, false);
+  auto y = __builtin_amdgcn_permlane32_swap(r1, r3, false, false);
+  auto u = __builtin_amdgcn_permlane16_swap(x[0], y[0], false, false);
+  auto v = __builtin_amdgcn_permlane16_swap(x[1], y[1], false, false);
+  r0 = u[0];
+  r1 = u[1];
+  r2 = v[0];
+  r3 = v[1];
+}
+__device__ __forceinline__ void lu_swap4(float &a, float &b, float &c, float &d) {
+  uint32_t x[4] = {__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), __float_as_uint(d)};
+  lu_swap4(x[0], x[1], x[2], x[3]);
+  a = __uint_as_float(x[0]);
+  b = __uint_as_float(x[1]);
+  c = __uint_as_float(x[2]);
+  d = __uint_as_float(x[3]);
+}
+__device__ __forceinline__ void lu_swap4(double &a, double &b, double &c, double &d) {
+  uint32_t l[4] = {(uint32_t)__double2loint(a), (uint32_t)__double2loint(b),
+                   (uint32_t)__double2loint(c), (uint32_t)__double2loint(d)};
+  uint32_t h[4] = {(uint32_t)__double2hiint(a), (uint32_t)__double2hiint(b),
+                   (uint32_t)__double2hiint(c), (uint32_t)__double2hiint(d)};
+  lu_swap4(l[0], l[1], l[2], l[3]);
+  lu_swap4(h[0], h[1], h[2], h[3]);
+  a = __hiloint2double((int)h[0], (int)l[0]);
+  b = __hiloint2double((int)h[1], (int)l[1]);
+  c = __hiloint2double((int)h[2], (int)l[2]);
+  d = __hiloint2double((int)h[3], (int)l[3]);
+}
 
+// 64 x 16 tile of the matrix as the matrix-core result of its transpose (row block g of 16:
+// lane l holds row 16 g + l % 16 and four columns), and back: between it and "lane = row,
+// register = column" the lane group trades places with one digit of the column.
+template <typename T>
+struct LuTile;
+template <>
+struct LuTile<float> {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  // column of register r of lane group c
+  static __device__ __forceinline__ int column(int c, int r) { return 4 * c + r; }
+  static __device__ __forceinline__ v4 mfma(float a, float b, v4 x) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, x, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void to_blocks(float (&x)[16], v4 (&m)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      lu_swap4(x[r], x[4 + r], x[8 + r], x[12 + r]);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) m[g][r] = x[4 * g + r];
+    }
+  }
+  static __device__ __forceinline__ void to_rows(const v4 (&m)[4], float (&x)[16]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) x[4 * g + r] = m[g][r];
+      lu_swap4(x[r], x[4 + r], x[8 + r], x[12 + r]);
+    }
+  }
+};
+template <>
+struct LuTile<double> {
+  typedef double v4 __attribute__((ext_vector_type(4)));
+  static __device__ __forceinline__ int column(int c, int r) { return 4 * r + c; }
+  static __device__ __forceinline__ v4 mfma(double a, double b, v4 x) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, x, 0, 0, 0);
+  }
+  static __device__ __forceinline__ void to_blocks(double (&x)[16], v4 (&m)[4]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      lu_swap4(x[4 * r], x[4 * r + 1], x[4 * r + 2], x[4 * r + 3]);
+#pragma unroll
+      for (int g = 0; g < 4; ++g) m[g][r] = x[4 * r + g];
+    }
+  }
+  static __device__ __forceinline__ void to_rows(const v4 (&m)[4], double (&x)[16]) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) x[4 * r + g] = m[g][r];
+      lu_swap4(x[4 * r], x[4 * r + 1], x[4 * r + 2], x[4 * r + 3]);
+    }
+  }
+};
+
+// Step P of a panel x[16] (lane = row): pivot by DPP arg-max, then every row takes f times
+// the pivot row away.  x[P] ends as f, and the multipliers of earlier steps are updated with
+// the rest, so that after the panel x holds the W of "row -= sum_p W[row][p] pivot row p of
+// the matrix before the panel".  The pivot row's half that holds P is broadcast by readlane,
+// the other half through LDS.
 template <int P, typename T>
-struct LuStep64 {
-  static __device__ __forceinline__ void run(T (&a)[64], int col, T &pivs, uint64_t &used,
-                                             int &parity, T *buf) {
-    // pivot key: |a| rounded to float with its 6 low mantissa bits replaced
-    // by 63 - lane (largest magnitude to 2^-17, then the lowest lane); NaN /
-    // Inf rank as 0
-    const T mag = fabs(a[P]);
+struct LuPanel {
+  static __device__ __forceinline__ void run(T (&x)[16], int col, T &pivs, uint64_t &used,
+                                             int &parity, int &step, T *buf) {
+    typedef LuVec<T> V;
+    const T mag = fabs(x[P]);
     const float fm = (mag <= lu_big<T>()) ? (float)mag : 0.0f;
     const uint32_t key = (__float_as_uint(fm) & ~63u) | (uint32_t)(63 - col);
     const int q = 63 - (int)(lu_wave_max(key) & 63u);
-    const T piv = lu_bcast(a[P], q);
     const bool mine = col == q;
+    constexpr int near = P & 8, far = 8 - near;
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < 8; j += V::n)
+        *reinterpret_cast<typename V::t *>(buf + j) = V::make(&x[far + j]);
+    }
+    const T piv = lu_bcast(x[P], q);
     pivs = mine ? piv : pivs;
-    if (P + 1 < 64) {
-      const T f = mine ? T(1) : lu_mult(a[P], piv);
-      typedef LuVec<T> V;
-      // entries [P + 1, js) by readlane, [js, 64) through LDS (js aligned)
-      constexpr int n_tail = ((63 - P) * V::tail6) / 6;
-      constexpr int js0 = (64 - n_tail + V::n - 1) & ~(V::n - 1);
-      constexpr int js = js0 < P + 1 ? ((P + 1 + V::n - 1) & ~(V::n - 1)) : js0;
-      if (js < 64 && mine) {
+    step = mine ? P : step;
+    const T f = mine ? T(1) : lu_mult(x[P], piv);
+    T r[8];
 #pragma unroll
-        for (int j = js; j < 64; j += V::n)
-          *reinterpret_cast<typename V::t *>(buf + j) = V::make(&a[j]);
-      }
-      // blocks of 8 readlane entries kept apart by scheduling barriers, so
-      // that the readlanes of one block are consumed before the next block's
-      // are issued (hoisting all of them overflows the scalar registers)
+    for (int j = 0; j < 8; ++j)
+      if (near + j != P) r[j] = lu_bcast(x[near + j], q);
 #pragma unroll
-      for (int j0 = P + 1; j0 < js && j0 < 64; j0 += 8) {
-        T r[8];
+    for (int j = 0; j < 8; ++j)
+      if (near + j != P) x[near + j] = fma(-f, r[j], x[near + j]);
+    x[P] = f;
+    wave_lds_fence();
 #pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (j0 + k < js && j0 + k < 64) r[k] = lu_bcast(a[j0 + k], q);
-#pragma unroll
-        for (int k = 0; k < 8; ++k)
-          if (j0 + k < js && j0 + k < 64) a[j0 + k] = fma(-f, r[k], a[j0 + k]);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      if (js < 64) {
-        wave_lds_fence();
-#pragma unroll
-        for (int j = js; j < 64; j += V::n) {
-          const typename V::t v = *reinterpret_cast<const typename V::t *>(buf + j);
-          a[j] = fma(-f, v.x, a[j]);
-          a[j + 1] = fma(-f, v.y, a[j + 1]);
-          if constexpr (V::n == 4) {
-            a[j + 2] = fma(-f, v.z, a[j + 2]);
-            a[j + 3] = fma(-f, v.w, a[j + 3]);
-          }
-        }
-        // the buffer is rewritten by the next step's pivot lane
-        wave_lds_fence();
+    for (int j = 0; j < 8; j += V::n) {
+      const typename V::t v = *reinterpret_cast<const typename V::t *>(buf + j);
+      x[far + j] = fma(-f, v.x, x[far + j]);
+      x[far + j + 1] = fma(-f, v.y, x[far + j + 1]);
+      if constexpr (V::n == 4) {
+        x[far + j + 2] = fma(-f, v.z, x[far + j + 2]);
+        x[far + j + 3] = fma(-f, v.w, x[far + j + 3]);
       }
     }
+    wave_lds_fence();
     // row exchanges: lanes chosen earlier with a higher index than q
     parity += __popcll(used & ~((2ull << q) - 1ull));
     used |= 1ull << q;
-    LuStep64<P + 1, T>::run(a, col, pivs, used, parity, buf);
+    LuPanel<P + 1, T>::run(x, col, pivs, used, parity, step, buf);
   }
 };
 
 template <typename T>
-struct LuStep64<64, T> {
-  static __device__ __forceinline__ void run(T (&)[64], int, T &, uint64_t &, int &, T *) {}
+struct LuPanel<16, T> {
+  static __device__ __forceinline__ void run(T (&)[16], int, T &, uint64_t &, int &, int &, T *) {}
 };
+
+// all four panels; the columns to the right of a panel are updated on the matrix cores
+template <typename T>
+__device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64_t &used,
+                                            int &parity, T *buf) {
+  typedef LuTile<T> L;
+  typedef typename L::v4 v4;
+  constexpr int LD = 20;      // LDS row of a tile of 16
+  const int c = col >> 4, x = col & 15;
+  T pan[16];
+  v4 tile[3][4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    T y[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) y[j] = a[16 * t + j];
+    if (t == 0) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) pan[j] = y[j];
+    } else {
+      L::to_blocks(y, tile[t - 1]);
+    }
+  }
+#pragma unroll 1
+  for (int k = 0; k < 4; ++k) {
+    int step = -1;
+    LuPanel<0, T>::run(pan, col, pivs, used, parity, step, buf);
+    if (k == 3) break;
+    v4 W[4];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) pan[j] = -pan[j];
+    L::to_blocks(pan, W);
+    uint32_t rk[4] = {(uint32_t)step, (uint32_t)step, (uint32_t)step, (uint32_t)step};
+    lu_swap4(rk[0], rk[1], rk[2], rk[3]);   // step of row 16 g + x
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (t < 3 - k) {
+        // the panel's pivot rows of the tile, as the left operand
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          if ((int)rk[g] >= 0) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) buf[(int)rk[g] * LD + L::column(c, r)] = tile[t][g][r];
+          }
+        wave_lds_fence();
+        T u[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) u[r] = buf[L::column(c, r) * LD + x];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) tile[t][g] = L::mfma(u[r], W[g][r], tile[t][g]);
+        wave_lds_fence();
+      }
+    }
+    L::to_rows(tile[0], pan);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      tile[0][g] = tile[1][g];
+      tile[1][g] = tile[2][g];
+    }
+  }
+}
 
 // sign and log|det| from the 64 pivots (lane l: the pivot taken from lane
 // l), summed in FP64 over the wave; a zero, non-finite or missing pivot
@@ -379,7 +516,8 @@ __device__ __forceinline__ GJResult lu_logdet(T (&a)[NFP], int col, int gbase, T
     T pivs = T(0);
     uint64_t used = 0ull;
     int parity = 0;
-    LuStep64<0, T>::run(a, col, pivs, used, parity, prow);
+    __shared__ __align__(16) T buf[8][16 * 20];   // (callers: at most eight waves)
+    lu64_panels<T>(a, col, pivs, used, parity, buf[threadIdx.x >> 6]);
     GJResult r{0.0, 0, false, -1};
     lu64_finish(pivs, used, parity, r.logdet, r.parity, r.singular);
     return r;

@@ -16,6 +16,8 @@
 // time; z1 is carried per walker and updated by the W1 columns of the moved
 // electrons, so only the two dense layers and the determinant are recomputed
 // per proposal.
+#include <type_traits>
+
 #include <hip/hip_bf16.h>
 #include <rocblas/rocblas.h>
 
@@ -120,38 +122,79 @@ __global__ void __launch_bounds__(256)
 }
 
 // ------------------------------------------------------------ determinant
+// list[j] = the j-th occupied orbital (up, then down, ascending), -1 beyond the electrons;
+// list: NFP ints of LDS private to the group
+template <int NFP>
+__device__ __forceinline__ void orbital_list(uint64_t up, uint64_t dn, int N, int col, int *list) {
+  list[col] = -1;
+  wave_lds_fence();
+  const int nu = __popcll(up);
+  for (int s = col; s < N; s += NFP) {
+    const uint64_t below = (1ull << s) - 1;
+    const int ku = __popcll(up & below), kd = nu + __popcll(dn & below);
+    if (((up >> s) & 1) && ku < NFP) list[ku] = s;
+    if (((dn >> s) & 1) && kd < NFP) list[kd] = N + s;
+  }
+  wave_lds_fence();
+}
+
+// The orbitals of rows j0 .. j0 + R - 1 of a group's matrix, handed to f:
+// the orbitals first, so that the loads that f makes are in flight together (with a branch
+// per row on the occupation masks each row waited for its own: 54184 matrices of 32 x 32 in
+// FP64 571 us, now 387).  R rows at a time: as many as leave the elimination its registers
+// (n_f = 64 in FP64, 8 rows: one wave per SIMD, and the inverses of nnbf_det_kernel 645 us
+// where 4 rows take 431).
+template <int NFP, int R, typename F>
+__device__ __forceinline__ void row_orbitals(const int *list, int j0, F f) {
+  int orb[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    orb[k] = list[j0 + k];
+    if constexpr (NFP == 64) orb[k] = __builtin_amdgcn_readfirstlane(orb[k]);
+  }
+  f(orb);
+  if constexpr (NFP == 64) __builtin_amdgcn_sched_barrier(0);   // (all 64 rows' loads spill)
+}
+
 // Builds A^T row-per-lane: a[j] = A[j][col] = M[orb_j][col] + s (D[orb_j*nf+col]
 // + bout[...]) for orb_j the j-th occupied orbital (ascending), with the
-// occupation masks given explicitly (up, dn).
+// occupation masks given explicitly (up, dn); list as orbital_list.
 // (bout NULL: Drow is the compact [nf][nf] of the occupied orbitals, biases added)
 template <int NFP, typename TW>
 __device__ __forceinline__ void nnbf_rows(double (&a)[NFP], uint64_t up, uint64_t dn, int N,
                                           int nf, int col, const TW *__restrict__ M,
                                           const TW *__restrict__ Drow,
-                                          const TW *__restrict__ bout, double s) {
-  uint64_t mu = up, md = dn;
+                                          const TW *__restrict__ bout, double s, int *list) {
+  orbital_list<NFP>(up, dn, N, col, list);
+  constexpr int R = NFP == 64 ? 4 : NFP < 16 ? 8 : 16;
+  const int c = col < nf ? col : 0;
+  auto rows = [&](auto compact) {
 #pragma unroll
-  for (int j = 0; j < NFP; ++j) {
-    int orb = -1;
-    if (mu) {
-      orb = __ffsll((long long)mu) - 1;
-      mu &= mu - 1;
-    } else if (md) {
-      orb = N + __ffsll((long long)md) - 1;
-      md &= md - 1;
+    for (int j0 = 0; j0 < NFP; j0 += R) {
+      row_orbitals<NFP, R>(list, j0, [&](const int (&orb)[R]) {
+        TW m[R], d[R], b[R];
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+          const int e = (orb[k] < 0 ? 0 : orb[k]) * nf + c;
+          m[k] = M[e];
+          d[k] = compact ? Drow[(j0 + k < nf ? j0 + k : 0) * nf + c] : Drow[e];
+          b[k] = compact ? TW(0) : bout[e];
+        }
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+          const int j = j0 + k;
+          const double v =
+              (double)m[k] + s * (compact ? (double)d[k] : (double)d[k] + (double)b[k]);
+          a[j] = j < nf && col < nf ? (orb[k] >= 0 ? v : 0.0) : (j == col ? 1.0 : 0.0);
+        }
+      });
     }
-    if (j < nf && col < nf) {
-      if (orb >= 0) {
-        const int64_t e = (int64_t)orb * nf + col;
-        a[j] = (double)M[e] + s * (bout ? (double)Drow[e] + (double)bout[e]
-                                        : (double)Drow[(int64_t)j * nf + col]);
-      } else {
-        a[j] = 0.0;
-      }
-    } else {
-      a[j] = (j == col) ? 1.0 : 0.0;
-    }
-  }
+  };
+  if (bout)
+    rows(std::false_type{});
+  else
+    rows(std::true_type{});
+  wave_lds_fence();   // the list's memory is the elimination's
 }
 
 template <int NFP>
@@ -176,7 +219,7 @@ __device__ __forceinline__ void group_masks(const int64_t *cfg, int N, int col, 
 
 // INV: also write A^-1 (Gauss-Jordan); otherwise the determinant only (LU)
 template <int NFP, bool INV, typename TW>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, NFP == 64 ? 2 : 1)
     nnbf_det_kernel(int64_t Bc, int N, int nf, const int64_t *__restrict__ cfg,
                     const TW *__restrict__ D, const TW *__restrict__ M,
                     const TW *__restrict__ bout, double s, double *sign,
@@ -196,7 +239,8 @@ __global__ void __launch_bounds__(256)
   const bool count_ok = (__popcll(up) + __popcll(dn)) == nf;
   double a[NFP];
   nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M,
-                     D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s);
+                     D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s,
+                     reinterpret_cast<int *>(prow));
   const bool nonfinite = group_nonfinite<NFP>(a, grp * NFP);
   const GJResult r = INV ? gj_invert<NFP>(a, col, grp * NFP, prow, qbuf)
                          : lu_logdet<NFP>(a, col, grp * NFP, prow);
@@ -639,7 +683,7 @@ __global__ void __launch_bounds__(NG2_T)
 // TL: the elimination's type (double; float for the FP32 determinant of the
 // mixed-precision amplitude, whose entries are formed by one FP32 fma)
 template <int NFP, typename TL>
-__global__ void __launch_bounds__(256)
+__global__ void __launch_bounds__(256, NFP == 64 ? (sizeof(TL) == 4 ? 4 : 2) : 1)
     nnbf_detA_kernel(int64_t Bc, int N, int nf, const int64_t *__restrict__ cfg,
                      const float *__restrict__ A, const float *__restrict__ M, double s,
                      double *sign, double *logabs) {
@@ -667,28 +711,32 @@ __global__ void __launch_bounds__(256)
   // FP32 elimination: the entries as fmaf(s, Docc, M), one rounding
   const float sf = (float)s;
   TL a[NFP];
-  uint64_t mu = up, md = dn;
+  int *list = reinterpret_cast<int *>(prow);
+  orbital_list<NFP>(up, dn, N, col, list);
+  constexpr int R = NFP < 16 || NFP == 64 ? 8 : 16;
+  const int c = col < nf ? col : 0;
 #pragma unroll
-  for (int j = 0; j < NFP; ++j) {
-    int orb = -1;
-    if (mu) {
-      orb = __ffsll((long long)mu) - 1;
-      mu &= mu - 1;
-    } else if (md) {
-      orb = N + __ffsll((long long)md) - 1;
-      md &= md - 1;
-    }
-    if (j < nf && col < nf) {
-      if (orb < 0)
-        a[j] = TL(0);
-      else if constexpr (sizeof(TL) == 4)
-        a[j] = fmaf(sf, Aw[(int64_t)j * nf + col], M[(int64_t)orb * nf + col]);
-      else
-        a[j] = (double)M[(int64_t)orb * nf + col] + s * (double)Aw[(int64_t)j * nf + col];
-    } else {
-      a[j] = (j == col) ? TL(1) : TL(0);
-    }
+  for (int j0 = 0; j0 < NFP; j0 += R) {
+    row_orbitals<NFP, R>(list, j0, [&](const int (&orb)[R]) {
+      float m[R], d[R];
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        m[k] = M[(int64_t)(orb[k] < 0 ? 0 : orb[k]) * nf + c];
+        d[k] = Aw[(int64_t)(j0 + k < nf ? j0 + k : 0) * nf + c];
+      }
+#pragma unroll
+      for (int k = 0; k < R; ++k) {
+        const int j = j0 + k;
+        TL v;
+        if constexpr (sizeof(TL) == 4)
+          v = fmaf(sf, d[k], m[k]);
+        else
+          v = (double)m[k] + s * (double)d[k];
+        a[j] = j < nf && col < nf ? (orb[k] >= 0 ? v : TL(0)) : (j == col ? TL(1) : TL(0));
+      }
+    });
   }
+  wave_lds_fence();   // the list's memory is the elimination's
   const bool nonfinite = group_nonfinite<NFP>(a, grp * NFP);
   const GJResult r = lu_logdet<NFP>(a, col, grp * NFP, prow);
   const bool singular = r.singular || !count_ok;
@@ -1109,8 +1157,10 @@ __global__ void masked_rows_kernel(int64_t B, int64_t row_words, const uint8_t *
 
 // Determinant of the proposed configuration, Metropolis test, commit; then the walker's
 // proposal on the next edge (if `more`).  The commit's columns of W1 are read from the
-// transposed weights, eight of a lane's units in flight (read by rows of W1, one unit at a
-// time, they were a third of the kernel's latency; TACC).
+// transposed weights, eight of a lane's units in flight.
+// Bound by the latency of one elimination (lu_logdet).  Measured, FP64: 6x6 (n_f = 32), 4096
+// walkers 38 us; 8x8 (n_f = 64), 1000 walkers 38 us (45.8 and 64 with a branch per row of the
+// matrix and the unblocked elimination).
 template <int NFP, typename TW>
 __global__ void __launch_bounds__(256)
     nnbf_accept_kernel(int64_t B, int N, int nf, int H, int i, int j, int64_t *cfg,
@@ -1139,7 +1189,8 @@ __global__ void __launch_bounds__(256)
          ((uint64_t)(nj & 1) << j);
     double a[NFP];
     nnbf_rows<NFP, TW>(a, up, dn, N, nf, col, M,
-                       D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s);
+                       D + w * (int64_t)nf * (bout ? 2 * N : nf), bout, s,
+                     reinterpret_cast<int *>(prow));
     const GJResult r = lu_logdet<NFP>(a, col, grp * NFP, prow);
     const double lp = r.singular ? log(1e-45) : fmax(r.logdet, log(1e-45));
     const double ratio = exp(2.0 * (lp - logabs[w]));

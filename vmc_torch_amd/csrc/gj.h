@@ -246,7 +246,7 @@ struct LuStep<NFP, NFP, T> {
   static __device__ __forceinline__ void run(T (&)[NFP], int, int, T *, LuState &) {}
 };
 
-// One 64 x 64 matrix per wave, in four panels of 16 columns: the panel is eliminated with a
+// One 64 x 64 FP64 matrix per wave, in four panels of 16 columns: the panel is eliminated with a
 // row per lane, the columns right of it take the panel's update on the matrix cores, in
 // between in the matrix-core result layout.  Every lane applies every step, the pivot lane
 // with multiplier exactly 1: its row becomes exact zeros, so a lane once chosen keys at most
@@ -258,8 +258,8 @@ struct LuStep<NFP, NFP, T> {
 // Bound by the vector instructions and the dependent chain of the 64 pivot searches.  A
 // step of the unblocked elimination updates up to 63 entries of a lane with up to 63
 // broadcasts, and its 64 unrolled steps exceed the instruction cache; here it is 15 and 15,
-// and the four panels share one code.  Measured, with the loads of nnbf_detA_kernel: 65536
-// FP32 determinants 707 -> 502 us; one wave's FP64 determinant in nnbf_accept_kernel 64 -> 38 us.
+// and the four panels share one code.  Measured: one wave's FP64 determinant, with its loads,
+// in nnbf_accept_kernel 64 -> 38 us.
 // multiplier a / piv: FP32 by the hardware reciprocal (1 ulp), FP64 by the
 // correctly rounded division
 __device__ __forceinline__ float lu_mult(float a, float piv) {
@@ -273,7 +273,7 @@ struct LuVec;
 template <>
 struct LuVec<float> {
   typedef float4 t;
-  static constexpr int n = 4;
+  static constexpr int n = 4, tail6 = 4;
   static __device__ __forceinline__ t make(const float *x) {
     return make_float4(x[0], x[1], x[2], x[3]);
   }
@@ -281,7 +281,7 @@ struct LuVec<float> {
 template <>
 struct LuVec<double> {
   typedef double2 t;
-  static constexpr int n = 2;
+  static constexpr int n = 2, tail6 = 3;
   static __device__ __forceinline__ t make(const double *x) { return make_double2(x[0], x[1]); }
 };
 // Exchange of register blocks and lane groups: reg[c] of lane group g <-> reg[g] of lane
@@ -295,14 +295,6 @@ __device__ __forceinline__ void lu_swap4(uint32_t &r0, uint32_t &r1, uint32_t &r
   r1 = u[1];
   r2 = v[0];
   r3 = v[1];
-}
-__device__ __forceinline__ void lu_swap4(float &a, float &b, float &c, float &d) {
-  uint32_t x[4] = {__float_as_uint(a), __float_as_uint(b), __float_as_uint(c), __float_as_uint(d)};
-  lu_swap4(x[0], x[1], x[2], x[3]);
-  a = __uint_as_float(x[0]);
-  b = __uint_as_float(x[1]);
-  c = __uint_as_float(x[2]);
-  d = __uint_as_float(x[3]);
 }
 __device__ __forceinline__ void lu_swap4(double &a, double &b, double &c, double &d) {
   uint32_t l[4] = {(uint32_t)__double2loint(a), (uint32_t)__double2loint(b),
@@ -322,31 +314,6 @@ __device__ __forceinline__ void lu_swap4(double &a, double &b, double &c, double
 // register = column" the lane group trades places with one digit of the column.
 template <typename T>
 struct LuTile;
-template <>
-struct LuTile<float> {
-  typedef float v4 __attribute__((ext_vector_type(4)));
-  // column of register r of lane group c
-  static __device__ __forceinline__ int column(int c, int r) { return 4 * c + r; }
-  static __device__ __forceinline__ v4 mfma(float a, float b, v4 x) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, x, 0, 0, 0);
-  }
-  static __device__ __forceinline__ void to_blocks(float (&x)[16], v4 (&m)[4]) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      lu_swap4(x[r], x[4 + r], x[8 + r], x[12 + r]);
-#pragma unroll
-      for (int g = 0; g < 4; ++g) m[g][r] = x[4 * g + r];
-    }
-  }
-  static __device__ __forceinline__ void to_rows(const v4 (&m)[4], float (&x)[16]) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-#pragma unroll
-      for (int g = 0; g < 4; ++g) x[4 * g + r] = m[g][r];
-      lu_swap4(x[r], x[4 + r], x[8 + r], x[12 + r]);
-    }
-  }
-};
 template <>
 struct LuTile<double> {
   typedef double v4 __attribute__((ext_vector_type(4)));
@@ -492,6 +459,81 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
   }
 }
 
+// FP32: unblocked.  The panels' update, formed from the pivot rows as they were before the
+// panel, loses a little to cancellation (median error of ln|det| 6 %, 99th percentile 10 to
+// 20 % above this one, over 8192 configurations at n_f = 36 to 64); in FP64 the two agree
+// (medians 7.4e-15 and 7.6e-15 against extended precision at n_f = 64).
+// The pivot row reaches the other lanes by readlane (its head: two vector instructions per
+// entry with the update) and through the wave's LDS buffer (its tail, 4/6: one), the split
+// that keeps both pipes busy.
+template <int P, typename T>
+struct LuStep64 {
+  static __device__ __forceinline__ void run(T (&a)[64], int col, T &pivs, uint64_t &used,
+                                             int &parity, T *buf) {
+    // pivot key: |a| rounded to float with its 6 low mantissa bits replaced
+    // by 63 - lane (largest magnitude to 2^-17, then the lowest lane); NaN /
+    // Inf rank as 0
+    const T mag = fabs(a[P]);
+    const float fm = (mag <= lu_big<T>()) ? (float)mag : 0.0f;
+    const uint32_t key = (__float_as_uint(fm) & ~63u) | (uint32_t)(63 - col);
+    const int q = 63 - (int)(lu_wave_max(key) & 63u);
+    const T piv = lu_bcast(a[P], q);
+    const bool mine = col == q;
+    pivs = mine ? piv : pivs;
+    if (P + 1 < 64) {
+      const T f = mine ? T(1) : lu_mult(a[P], piv);
+      typedef LuVec<T> V;
+      // entries [P + 1, js) by readlane, [js, 64) through LDS (js aligned)
+      constexpr int n_tail = ((63 - P) * V::tail6) / 6;
+      constexpr int js0 = (64 - n_tail + V::n - 1) & ~(V::n - 1);
+      constexpr int js = js0 < P + 1 ? ((P + 1 + V::n - 1) & ~(V::n - 1)) : js0;
+      if (js < 64 && mine) {
+#pragma unroll
+        for (int j = js; j < 64; j += V::n)
+          *reinterpret_cast<typename V::t *>(buf + j) = V::make(&a[j]);
+      }
+      // blocks of 8 readlane entries kept apart by scheduling barriers, so
+      // that the readlanes of one block are consumed before the next block's
+      // are issued (hoisting all of them overflows the scalar registers)
+#pragma unroll
+      for (int j0 = P + 1; j0 < js && j0 < 64; j0 += 8) {
+        T r[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (j0 + k < js && j0 + k < 64) r[k] = lu_bcast(a[j0 + k], q);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+          if (j0 + k < js && j0 + k < 64) a[j0 + k] = fma(-f, r[k], a[j0 + k]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (js < 64) {
+        wave_lds_fence();
+#pragma unroll
+        for (int j = js; j < 64; j += V::n) {
+          const typename V::t v = *reinterpret_cast<const typename V::t *>(buf + j);
+          a[j] = fma(-f, v.x, a[j]);
+          a[j + 1] = fma(-f, v.y, a[j + 1]);
+          if constexpr (V::n == 4) {
+            a[j + 2] = fma(-f, v.z, a[j + 2]);
+            a[j + 3] = fma(-f, v.w, a[j + 3]);
+          }
+        }
+        // the buffer is rewritten by the next step's pivot lane
+        wave_lds_fence();
+      }
+    }
+    // row exchanges: lanes chosen earlier with a higher index than q
+    parity += __popcll(used & ~((2ull << q) - 1ull));
+    used |= 1ull << q;
+    LuStep64<P + 1, T>::run(a, col, pivs, used, parity, buf);
+  }
+};
+
+template <typename T>
+struct LuStep64<64, T> {
+  static __device__ __forceinline__ void run(T (&)[64], int, T &, uint64_t &, int &, T *) {}
+};
+
 // sign and log|det| from the 64 pivots (lane l: the pivot taken from lane
 // l), summed in FP64 over the wave; a zero, non-finite or missing pivot
 // (a lane never chosen keeps 0) makes the matrix singular
@@ -516,8 +558,12 @@ __device__ __forceinline__ GJResult lu_logdet(T (&a)[NFP], int col, int gbase, T
     T pivs = T(0);
     uint64_t used = 0ull;
     int parity = 0;
-    __shared__ __align__(16) T buf[8][16 * 20];   // (callers: at most eight waves)
-    lu64_panels<T>(a, col, pivs, used, parity, buf[threadIdx.x >> 6]);
+    if constexpr (sizeof(T) == 4) {
+      LuStep64<0, T>::run(a, col, pivs, used, parity, prow);
+    } else {
+      __shared__ __align__(16) T buf[8][16 * 20];   // (callers: at most eight waves)
+      lu64_panels<T>(a, col, pivs, used, parity, buf[threadIdx.x >> 6]);
+    }
     GJResult r{0.0, 0, false, -1};
     lu64_finish(pivs, used, parity, r.logdet, r.parity, r.singular);
     return r;

@@ -9,17 +9,23 @@
 // device flag set on convergence turns every later launch of the loop into
 // an immediate return, so the host never waits inside the solve.
 //
-// Per iteration three launches (four when Np > 8192):
-//   mr_apply      inner = O v and the row-chunk sums of O^T inner from ONE read of O
-//                 (a workgroup keeps its rows and its sums in registers; Np > 8192:
-//                 mr_gemv_rows, then mr_colsum_partial, two reads), and, in workgroups
-//                 of their own, Obar . v and the previous iteration's x update and
-//                 convergence test;
-//   mr_form_y     the chunk sums added up, y, and v . y per block;
-//   mr_finish     alfa, the orthogonalised y, ||y||, the Givens rotation.
-// A launch of this size costs 2 - 3 us whatever it does, so the count of launches bounds
-// small and medium problems: at Ns = 2900, Np = 2160 an iteration takes 17 us (measured);
-// 15 launches and two reads of O took 45 to 67.
+// The update is not determined by its inputs alone at the usual settings (heavy-tailed O,
+// shift 1e-2): the Lanczos vectors lose their orthogonality, and another order of the sums
+// gives an update that differs by per cents.  So every sum has one order, whatever the
+// form: products and vector sums by one fma chain per thread of the blocks of
+// mr_dot_partial / mr_gemv_rows, then trees; column sums over kRowChunks row chunks.
+//
+// Per iteration, up to kNarrowNp parameters, four launches:
+//   mr_rows        inner = O v (256 threads a row), and, in workgroups of their own,
+//                  Obar . v and the previous iteration's x update and convergence test;
+//   mr_colsum_partial   the row-chunk sums of O^T inner;
+//   mr_form_y_narrow    the chunk sums added up, and y;
+//   mr_finish      alfa, the orthogonalised y, ||y||, the Givens rotation (one workgroup).
+// A launch costs 2 - 3 us whatever it does, so the count of launches bounds small and
+// medium problems: a solve of 2900 samples and 2160 parameters, 100 iterations launched and
+// a third of them made, takes 2.2 ms, of 516 and 480 1.4 ms (15 launches: 4.6 to 6.2 and 6.0;
+// the same bits).  Above kNarrowNp the length-Np work takes the whole chip, in 15
+// launches: one workgroup would walk 53 MB an iteration at 2.2 M parameters.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -40,16 +46,15 @@ struct Neu2 {
 };
 
 constexpr int kRowChunks = 64;     // row chunks of the O^T w column sums
-constexpr int kApplyChunks = 2 * kRowChunks;  // row chunks of mr_apply (one workgroup each):
-                                              // as many sums as the two kept before
-constexpr int64_t kApplyNp = 8192; // widest row of mr_apply (8 columns a thread)
-constexpr int kDotBlocks = 1024;   // first-stage blocks of a length-Np dot
+constexpr int kDotBlocks = 1024;   // first-stage blocks of a length-Np dot (one per 2048)
+constexpr int kNarrowBlocks = 4;   // first-stage blocks that one workgroup of 1024 stands for
+constexpr int64_t kNarrowNp = 2048 * kNarrowBlocks;
 
 // scalar slots
 enum {
   S_BETA = 0, S_OLDB, S_ALFA, S_CS, S_SN, S_DBAR, S_EPSLN, S_PHIBAR, S_ANORM2, S_OLDEPS,
   S_DELTA, S_GAMMA, S_PHI, S_DONE, S_ITN, S_MV, S_YNORM2, S_BETA2, S_BNORM2, S_INFO,
-  S_EMEAN, S_EVAR, S_ZERO = 31, S_COUNT = 32
+  S_EMEAN, S_EVAR, S_STOP, S_ZERO = 31, S_COUNT = 32
 };
 
 __global__ void __launch_bounds__(256)
@@ -172,28 +177,144 @@ __global__ void mr_init(double *sc, int maxiter) {
   sc[S_PHIBAR] = bn;
   sc[S_INFO] = (double)maxiter;
   if (bn == 0.0) {
+    sc[S_STOP] = 1.0;
     sc[S_DONE] = 1.0;
     sc[S_INFO] = 0.0;
   }
 }
 
-// block-wide sums of NV values (512 or 1024 threads), the same in every thread
-template <int NT, int NV>
-__device__ __forceinline__ void block_sums(double (&v)[NV], double (*sh)[NT / 64]) {
-#pragma unroll
-  for (int i = 0; i < NV; ++i)
-    for (int o = 32; o > 0; o >>= 1) v[i] += __shfl_xor(v[i], o, 64);
-  if ((threadIdx.x & 63) == 0)
-#pragma unroll
-    for (int i = 0; i < NV; ++i) sh[i][threadIdx.x >> 6] = v[i];
-  __syncthreads();
-#pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    double t = 0.0;
-#pragma unroll
-    for (int k = 0; k < NT / 64; ++k) t += sh[i][k];
-    v[i] = t;
+// the Givens rotation of the new Lanczos column, beta = ||y|| (one thread)
+__device__ void mr_rotate_step(double alfa, double oldb, double beta, double *sc) {
+  const double cs = sc[S_CS], sn = sc[S_SN], dbar = sc[S_DBAR], phibar = sc[S_PHIBAR];
+  sc[S_OLDB] = oldb;
+  sc[S_BETA] = beta;
+  sc[S_OLDEPS] = sc[S_EPSLN];
+  sc[S_DELTA] = fma(alfa, sn, cs * dbar);
+  const double gbar = fma(sn, dbar, -(cs * alfa));
+  sc[S_EPSLN] = sn * beta;
+  sc[S_DBAR] = -cs * beta;
+  double gamma = sqrt(fma(beta, beta, gbar * gbar));
+  gamma = gamma > 1e-300 ? gamma : 1e-300;
+  sc[S_GAMMA] = gamma;
+  const double ncs = gbar / gamma, nsn = beta / gamma;
+  sc[S_CS] = ncs;
+  sc[S_SN] = nsn;
+  sc[S_PHI] = ncs * phibar;
+  sc[S_PHIBAR] = nsn * phibar;
+  sc[S_ANORM2] += fma(beta, beta, fma(alfa, alfa, oldb * oldb));
+}
+
+// the convergence test after an update of x (one thread)
+__device__ void mr_test(double rtol, double ynorm2, int flag, double *sc) {
+  sc[S_ITN] += 1.0;
+  const double rnorm = fabs(sc[S_PHIBAR]);
+  if (rnorm < rtol * sqrt(sc[S_ANORM2]) * sqrt(ynorm2) || sc[S_BETA] == 0.0) {
+    sc[flag] = 1.0;
+    sc[S_INFO] = 0.0;
   }
+}
+
+// ------------------------------------------------------------ Np > kNarrowNp
+// v[s] = sum_p O[s][p] x[p]
+__global__ void __launch_bounds__(256)
+    mr_gemv_rows(int64_t Np, const void *O, int o_dtype, int64_t ldo, const double *x,
+                 double *v, const double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  __shared__ double sh[4];
+  const int64_t s = blockIdx.x;
+  double acc = 0.0;
+  if (o_dtype == 0) {
+    const double *row = (const double *)O + s * ldo;
+    for (int64_t p = threadIdx.x; p < Np; p += blockDim.x) acc = fma(row[p], x[p], acc);
+  } else {
+    const float *row = (const float *)O + s * ldo;
+    for (int64_t p = threadIdx.x; p < Np; p += blockDim.x) acc = fma((double)row[p], x[p], acc);
+  }
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0) v[s] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// v = r2 / beta
+__global__ void mr_scale_v(int64_t n, const double *r2, double *v, const double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  const double s = 1.0 / sc[S_BETA];
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) v[i] = s * r2[i];
+}
+
+// y = Sx - (Obar . v) Obar + shift v - (beta / oldb) r1   (last term after
+// the first iteration)
+__device__ __forceinline__ double mr_y(double sx, double m, double v, double r1, double shift,
+                                       double mv, double c) {
+  const double t = fma(shift, v, fma(-mv, m, sx));
+  return c != 0.0 ? fma(-c, r1, t) : t;
+}
+__global__ void mr_form_y(int64_t n, const double *Sx, const double *m, const double *v,
+                          const double *r1, double shift, double *y, const double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  const double c = sc[S_ITN] >= 1.0 ? sc[S_BETA] / sc[S_OLDB] : 0.0;
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i] = mr_y(Sx[i], m[i], v[i], r1[i], shift, sc[S_MV], c);
+}
+
+// y -= (alfa / beta) r2
+__global__ void mr_orth_y(int64_t n, const double *r2, double *y, const double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  const double c = sc[S_ALFA] / sc[S_BETA];
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) y[i] = fma(-c, r2[i], y[i]);
+}
+
+__global__ void mr_rotate(double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  mr_rotate_step(sc[S_ALFA], sc[S_BETA], sqrt(sc[S_BETA2]), sc);
+}
+
+// w = (v - oldeps w1 - delta w2) / gamma, x += phi w
+struct MrStep {
+  double oe, de, ig, ph;
+};
+__device__ __forceinline__ MrStep mr_step(const double *sc) {
+  return {sc[S_OLDEPS], sc[S_DELTA], 1.0 / sc[S_GAMMA], sc[S_PHI]};
+}
+__device__ __forceinline__ double mr_w(const MrStep &c, double v, double w1, double w2) {
+  return fma(-c.de, w2, fma(-c.oe, w1, v)) * c.ig;
+}
+__global__ void mr_update_x(int64_t n, const double *v, const double *w1, const double *w2,
+                            double *w, double *x, const double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  const MrStep c = mr_step(sc);
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    const double wi = mr_w(c, v[i], w1[i], w2[i]);
+    w[i] = wi;
+    x[i] = fma(c.ph, wi, x[i]);
+  }
+}
+
+__global__ void mr_check(double rtol, double *sc) {
+  if (sc[S_DONE] != 0.0) return;
+  mr_test(rtol, sc[S_YNORM2], S_DONE, sc);
+}
+
+// ------------------------------------------------------------ Np <= kNarrowNp
+// The sum of a length-n dot's per-thread parts in a workgroup of 1024, which stands for the
+// nb blocks of mr_dot_partial (thread t: thread t % 256 of block t / 256, elements from
+// 256 (t / 256) + t % 256 = t in steps of 256 nb) and for mr_dot_final.  The same in every
+// thread.
+__device__ __forceinline__ double mr_total(double acc, int nb, double *sh) {
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+  if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  double p[kNarrowBlocks];
+#pragma unroll
+  for (int b = 0; b < kNarrowBlocks; ++b)
+    p[b] = b < nb ? (sh[4 * b] + sh[4 * b + 1]) + (sh[4 * b + 2] + sh[4 * b + 3]) : 0.0;
+  Neu2 a;
+  a.add((p[0] + p[2]) + (p[1] + p[3]));
+  return a.s + a.c;
 }
 
 struct MrVecs {
@@ -203,222 +324,116 @@ struct MrVecs {
   int first;                   // no last iteration
 };
 
-// Obar . v (one workgroup)
-template <int NT>
-__device__ void mr_mean_dot(int64_t n, const MrVecs &q, double *sc, double (*sh)[NT / 64]) {
-  const double s = 1.0 / sc[S_BETA];
-  double a[1] = {0.0};
-  for (int64_t i = threadIdx.x; i < n; i += NT) a[0] += q.m[i] * (s * q.r2[i]);
-  block_sums<NT, 1>(a, sh);
-  if (threadIdx.x == 0) sc[S_MV] = a[0];
-}
-
-// w = (v - oldeps w1 - delta w2) / gamma, x += phi w with the last iteration's v, and its
-// convergence test (one workgroup)
-template <int NT>
-__device__ void mr_update_x(int64_t n, const MrVecs &q, double rtol, double *sc,
-                            double (*sh)[NT / 64]) {
-  const double oe = sc[S_OLDEPS], de = sc[S_DELTA], ig = 1.0 / sc[S_GAMMA], ph = sc[S_PHI];
+// the x update of an iteration, with v = r1 / oldb, and its convergence test into sc[flag]
+__device__ void mr_narrow_update(int n, int nb, const MrVecs &q, double rtol, int flag,
+                                 double *sc, double *sh) {
+  const MrStep c = mr_step(sc);
   const double s = 1.0 / sc[S_OLDB];
-  double a[1] = {0.0};
-  for (int64_t i = threadIdx.x; i < n; i += NT) {
-    const double wi = (s * q.r1[i] - oe * q.w1[i] - de * q.w2[i]) * ig;
-    q.w[i] = wi;
-    const double xi = q.x[i] + ph * wi;
-    q.x[i] = xi;
-    a[0] += xi * xi;
-  }
-  block_sums<NT, 1>(a, sh);
-  if (threadIdx.x == 0) {
-    sc[S_YNORM2] = a[0];
-    sc[S_ITN] += 1.0;
-    const double rnorm = fabs(sc[S_PHIBAR]);
-    if (rnorm < rtol * sqrt(sc[S_ANORM2]) * sqrt(a[0]) || sc[S_BETA] == 0.0) {
-      sc[S_DONE] = 1.0;
-      sc[S_INFO] = 0.0;
+  double a = 0.0;
+  if ((int)threadIdx.x < 256 * nb)
+    for (int i = threadIdx.x; i < n; i += 256 * nb) {
+      const double wi = mr_w(c, s * q.r1[i], q.w1[i], q.w2[i]);
+      q.w[i] = wi;
+      const double xi = fma(c.ph, wi, q.x[i]);
+      q.x[i] = xi;
+      a = fma(xi, xi, a);
     }
-  }
+  a = mr_total(a, nb, sh);
+  if (threadIdx.x == 0) mr_test(rtol, a, flag, sc);
 }
 
-// inner = O v and the sums of O^T inner over this workgroup's rows from one read of O:
-// thread t holds the columns t, t + 1024, ... (E of them) of RB rows, of v and of the
-// compensated sums in registers; the next RB rows are loaded while the products of these
-// are summed over the workgroup (RB = 2 while that fits 128 registers: half the barriers).
-// Workgroups beyond the row chunks: Obar . v and the last x update (a flag that the latter
-// sets while the others run is seen by the next launch, which then ignores what they
-// wrote).
-template <int E, int RB, typename T>
+// inner = O v, four rows a workgroup; the first two workgroups: Obar . v and the last x
+// update.  That update's test sets S_STOP, which this launch does not read: S_DONE, which it
+// does, follows in mr_finish (waves of a workgroup that read a flag while it is set would
+// disagree on the way to their barrier).
 __global__ void __launch_bounds__(1024)
-    mr_apply(int64_t Ns, int64_t Np, const T *__restrict__ O, int64_t ldo, int64_t rows,
-             int chunks, MrVecs q, double rtol, double *__restrict__ partial, double *sc) {
+    mr_rows(int64_t Ns, int n, int nb, const void *O, int o_dtype, int64_t ldo, MrVecs q,
+            double rtol, double *inner, double *sc) {
   if (sc[S_DONE] != 0.0) return;
-  __shared__ double sh[2][RB][16];
+  __shared__ double sh[16];
   const int tid = threadIdx.x;
-  if ((int)blockIdx.x >= chunks) {
-    if ((int)blockIdx.x == chunks)
-      mr_mean_dot<1024>(Np, q, sc, sh[0]);
-    else if (!q.first)
-      mr_update_x<1024>(Np, q, rtol, sc, sh[0]);
-    return;
-  }
-  const int64_t r0 = blockIdx.x * rows, r1 = (r0 + rows < Ns) ? r0 + rows : Ns;
-  const double s = 1.0 / sc[S_BETA];
-  double v[E];
-  Neu2 acc[E];
-  T cur[RB][E], nxt[RB][E];
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int64_t p = tid + 1024 * (int64_t)e;
-    v[e] = p < Np ? s * q.r2[p] : 0.0;
-  }
-  auto load = [&](int64_t r, T (&d)[RB][E]) {
-#pragma unroll
-    for (int k = 0; k < RB; ++k)
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        const int64_t p = tid + 1024 * (int64_t)e;
-        d[k][e] = (r + k < r1 && p < Np) ? O[(r + k) * ldo + p] : (T)0;
-      }
-  };
-  load(r0, cur);
-  int buf = 0;
-  for (int64_t r = r0; r < r1; r += RB, buf ^= 1) {
-    load(r + RB, nxt);
-    double d[RB];
-#pragma unroll
-    for (int k = 0; k < RB; ++k) {
-      d[k] = 0.0;
-#pragma unroll
-      for (int e = 0; e < E; ++e) d[k] += (double)cur[k][e] * v[e];
-    }
-    block_sums<1024, RB>(d, sh[buf]);
-#pragma unroll
-    for (int k = 0; k < RB; ++k)
-#pragma unroll
-      for (int e = 0; e < E; ++e) {
-        acc[e].add((double)cur[k][e] * d[k]);
-        cur[k][e] = nxt[k][e];
-      }
-  }
-#pragma unroll
-  for (int e = 0; e < E; ++e) {
-    const int64_t p = tid + 1024 * (int64_t)e;
-    if (p < Np) partial[(int64_t)blockIdx.x * Np + p] = acc[e].s + acc[e].c;
-  }
-}
-
-// O v by rows when a row does not fit a workgroup's registers; the last two workgroups as
-// in mr_apply
-__global__ void __launch_bounds__(512)
-    mr_gemv_rows(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo, MrVecs q,
-                 double rtol, double *inner, double *sc) {
-  if (sc[S_DONE] != 0.0) return;
-  __shared__ double sh[1][8];
-  const int64_t s = blockIdx.x;
-  if (s >= Ns) {
-    if (s == Ns)
-      mr_mean_dot<512>(Np, q, sc, sh);
-    else if (!q.first)
-      mr_update_x<512>(Np, q, rtol, sc, sh);
-    return;
-  }
   const double is = 1.0 / sc[S_BETA];
-  double acc[1] = {0.0};
-  if (o_dtype == 0) {
-    const double *row = (const double *)O + s * ldo;
-    for (int64_t p = threadIdx.x; p < Np; p += 512) acc[0] += row[p] * (is * q.r2[p]);
-  } else {
-    const float *row = (const float *)O + s * ldo;
-    for (int64_t p = threadIdx.x; p < Np; p += 512) acc[0] += (double)row[p] * (is * q.r2[p]);
+  if (blockIdx.x == 1) {
+    if (!q.first) mr_narrow_update(n, nb, q, rtol, S_STOP, sc, sh);
+    return;
   }
-  block_sums<512, 1>(acc, sh);
-  if (threadIdx.x == 0) inner[s] = acc[0];
-}
-
-// y = S v - (Obar . v) Obar + shift v - (beta / oldb) r1 (last term after the first
-// iteration) from the chunk sums of O^T (O v), and the block's part of v . y: 16 columns
-// per block, 64 threads over the chunks of each
-__global__ void __launch_bounds__(1024)
-    mr_form_y(int64_t n, int chunks, const double *__restrict__ partial, double scale,
-              const double *__restrict__ m, const double *__restrict__ r1,
-              const double *__restrict__ r2, double shift, double *y, double *part,
-              const double *sc) {
-  if (sc[S_DONE] != 0.0) return;
-  __shared__ double sh[64][17];
-  const int col = threadIdx.x & 15, g = threadIdx.x >> 4;
-  const int64_t p = (int64_t)blockIdx.x * 16 + col;
-  Neu2 a;
-  if (p < n)
-    for (int c = g; c < chunks; c += 64) a.add(partial[(int64_t)c * n + p]);
-  sh[g][col] = a.s + a.c;
-  __syncthreads();
-  if (g < 4) {
-    Neu2 b;
-    for (int k = 0; k < 16; ++k) b.add(sh[g * 16 + k][col]);
-    // the four partial sums of a column sit in lanes 16 apart of the first wave
-    Neu2 t;
-    const double own = b.s + b.c;
-    for (int k = 0; k < 4; ++k) t.add(__shfl(own, k * 16 + col, 64));
-    double vy = 0.0;
-    if (g == 0 && p < n) {
-      const double v = r2[p] * (1.0 / sc[S_BETA]);
-      const double c = sc[S_ITN] >= 1.0 ? sc[S_BETA] / sc[S_OLDB] : 0.0;
-      double yi = (t.s + t.c) * scale - sc[S_MV] * m[p] + shift * v;
-      if (c != 0.0) yi -= c * r1[p];
-      y[p] = yi;
-      vy = v * yi;
+  double acc = 0.0;
+  if (blockIdx.x == 0) {
+    if (tid < 256 * nb)
+      for (int i = tid; i < n; i += 256 * nb) acc = fma(q.m[i], is * q.r2[i], acc);
+    acc = mr_total(acc, nb, sh);
+    if (tid == 0) sc[S_MV] = acc;
+    return;
+  }
+  const int64_t s = 4 * ((int64_t)blockIdx.x - 2) + (tid >> 8);
+  if (s < Ns) {
+    if (o_dtype == 0) {
+      const double *row = (const double *)O + s * ldo;
+#pragma unroll 4
+      for (int p = tid & 255; p < n; p += 256) acc = fma(row[p], is * q.r2[p], acc);
+    } else {
+      const float *row = (const float *)O + s * ldo;
+#pragma unroll 4
+      for (int p = tid & 255; p < n; p += 256) acc = fma((double)row[p], is * q.r2[p], acc);
     }
-    for (int o = 8; o > 0; o >>= 1) vy += __shfl_xor(vy, o, 64);
-    if (threadIdx.x == 0) part[blockIdx.x] = vy;
   }
+  for (int o = 32; o > 0; o >>= 1) acc += __shfl_down(acc, o, 64);
+  if ((tid & 63) == 0) sh[tid >> 6] = acc;
+  __syncthreads();
+  const int b = tid >> 6;
+  if ((tid & 255) == 0 && s < Ns) inner[s] = (sh[b] + sh[b + 1]) + (sh[b + 2] + sh[b + 3]);
 }
 
-// alfa = v . y, y -= (alfa / beta) r2, and the Givens rotation of the new Lanczos column
-// (one workgroup: a length-Np vector is a few us for one CU, as is another launch)
+// mr_colsum_final and mr_form_y
+__global__ void __launch_bounds__(64)
+    mr_form_y_narrow(int n, const double *__restrict__ partial, double scale,
+                     const double *__restrict__ m, const double *__restrict__ r1,
+                     const double *__restrict__ r2, double shift, double *y, const double *sc) {
+  if (sc[S_STOP] != 0.0) return;
+  const int p = blockIdx.x * 64 + threadIdx.x;
+  if (p >= n) return;
+  Neu2 a;
+#pragma unroll 16
+  for (int r = 0; r < kRowChunks; ++r) a.add(partial[(int64_t)r * n + p]);
+  const double c = sc[S_ITN] >= 1.0 ? sc[S_BETA] / sc[S_OLDB] : 0.0;
+  y[p] = mr_y((a.s + a.c) * scale, m[p], r2[p] * (1.0 / sc[S_BETA]), r1[p], shift, sc[S_MV], c);
+}
+
+// alfa = v . y, y -= (alfa / beta) r2, ||y|| and the Givens rotation (one workgroup: a vector
+// of this length is a few us for one CU, as is another launch)
 __global__ void __launch_bounds__(1024)
-    mr_finish(int64_t n, int64_t nb, const double *__restrict__ part,
-              const double *__restrict__ r2, double *y, double *sc) {
-  if (sc[S_DONE] != 0.0) return;
-  __shared__ double sh[2][1][16];
-  double a[1] = {0.0};
-  for (int64_t i = threadIdx.x; i < nb; i += 1024) a[0] += part[i];
-  block_sums<1024, 1>(a, sh[0]);
-  const double alfa = a[0], oldb = sc[S_BETA], c = alfa / oldb;
-  a[0] = 0.0;
-  for (int64_t i = threadIdx.x; i < n; i += 1024) {
-    const double yi = y[i] - c * r2[i];
-    y[i] = yi;
-    a[0] += yi * yi;
+    mr_finish(int n, int nb, const double *__restrict__ r2, double *y, double *sc) {
+  if (sc[S_STOP] != 0.0) {
+    if (threadIdx.x == 0) sc[S_DONE] = 1.0;
+    return;
   }
-  block_sums<1024, 1>(a, sh[1]);
-  if (threadIdx.x != 0) return;
-  const double beta = sqrt(a[0]);
-  const double cs = sc[S_CS], sn = sc[S_SN], dbar = sc[S_DBAR];
+  __shared__ double sh[2][16];
+  const int tid = threadIdx.x, step = 256 * nb;
+  const bool on = tid < step;
+  const double beta = sc[S_BETA], is = 1.0 / beta;
+  double a = 0.0;
+  if (on)
+    for (int i = tid; i < n; i += step) a = fma(is * r2[i], y[i], a);
+  const double alfa = mr_total(a, nb, sh[0]), c = alfa / beta;
+  a = 0.0;
+  if (on)
+    for (int i = tid; i < n; i += step) {
+      const double yi = fma(-c, r2[i], y[i]);
+      y[i] = yi;
+      a = fma(yi, yi, a);
+    }
+  a = mr_total(a, nb, sh[1]);
+  if (tid != 0) return;
   sc[S_ALFA] = alfa;
-  sc[S_OLDB] = oldb;
-  sc[S_BETA] = beta;
-  sc[S_OLDEPS] = sc[S_EPSLN];
-  sc[S_DELTA] = cs * dbar + sn * alfa;
-  const double gbar = sn * dbar - cs * alfa;
-  sc[S_EPSLN] = sn * beta;
-  sc[S_DBAR] = -cs * beta;
-  double gamma = sqrt(gbar * gbar + beta * beta);
-  gamma = gamma > 1e-300 ? gamma : 1e-300;
-  sc[S_GAMMA] = gamma;
-  const double ncs = gbar / gamma, nsn = beta / gamma;
-  sc[S_CS] = ncs;
-  sc[S_SN] = nsn;
-  sc[S_PHI] = ncs * sc[S_PHIBAR];
-  sc[S_PHIBAR] = nsn * sc[S_PHIBAR];
-  sc[S_ANORM2] += alfa * alfa + oldb * oldb + beta * beta;
+  mr_rotate_step(alfa, beta, sqrt(a), sc);
 }
 
 // the x update of the last iteration
-__global__ void __launch_bounds__(512) mr_last_update(int64_t n, MrVecs q, double rtol,
-                                                      double *sc) {
+__global__ void __launch_bounds__(1024)
+    mr_last_update(int n, int nb, MrVecs q, double rtol, double *sc) {
   if (sc[S_DONE] != 0.0) return;
-  __shared__ double sh[1][8];
-  mr_update_x<512>(n, q, rtol, sc, sh);
+  __shared__ double sh[16];
+  mr_narrow_update(n, nb, q, rtol, S_STOP, sc, sh);
 }
 
 // stats <- [mean E, var E, |phibar| (residual estimate), ||g||, iterations]
@@ -453,8 +468,7 @@ MrLayout mr_layout(int64_t Ns, int64_t Np) {
   L.w = take((size_t)Ns * 8);
   L.inner = take((size_t)Ns * 8);
   L.partial = take((size_t)2 * kRowChunks * Np * 8);
-  const size_t yblocks = (size_t)(Np + 15) / 16;
-  L.dotp = take((yblocks > kDotBlocks ? yblocks : kDotBlocks) * 8);
+  L.dotp = take((size_t)kDotBlocks * 8);
   L.sc = take((size_t)S_COUNT * 8);
   L.total = off;
   return L;
@@ -526,76 +540,79 @@ int sr_minres(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo, c
   hipLaunchKernelGGL(mr_zero, dim3(gn), dim3(256), 0, st, Np, w2);
   hipLaunchKernelGGL(mr_zero, dim3(gn), dim3(256), 0, st, Np, wn);
   VMCX_LAUNCHED();
-  // rows of a chunk: even (taken in pairs), all chunks in use
-  const int64_t arows = ((Ns + kApplyChunks - 1) / kApplyChunks + 1) & ~(int64_t)1;
-  const bool fused = Np <= kApplyNp;
-  const int chunks = fused ? (int)((Ns + arows - 1) / arows) : kRowChunks;
-  const unsigned yb = (unsigned)((Np + 15) / 16);
-  auto apply = [&](const MrVecs &q) {
-    const dim3 grid((unsigned)chunks + 2), block(1024);
-#define MR_APPLY(E, RB)                                                                         \
-  do {                                                                                          \
-    if (o_dtype == 0)                                                                           \
-      hipLaunchKernelGGL((mr_apply<E, RB, double>), grid, block, 0, st, Ns, Np,                 \
-                         (const double *)O, ldo, arows, chunks, q, rtol, partial, sc);          \
-    else                                                                                        \
-      hipLaunchKernelGGL((mr_apply<E, RB, float>), grid, block, 0, st, Ns, Np,                  \
-                         (const float *)O, ldo, arows, chunks, q, rtol, partial, sc);           \
-  } while (0)
-    const int64_t e = (Np + 1023) / 1024;
-    if (e <= 1)
-      MR_APPLY(1, 2);
-    else if (e <= 2)
-      MR_APPLY(2, 2);
-    else if (e <= 3)
-      MR_APPLY(3, 2);
-    else if (e <= 4)
-      MR_APPLY(4, 2);
-    else if (e <= 6)
-      MR_APPLY(6, 1);
-    else
-      MR_APPLY(8, 1);
-#undef MR_APPLY
-  };
-  MrVecs q{};
-  q.m = m;
-  q.x = x;
-  for (int it = 0; it < maxiter; ++it) {
-    q.r1 = r1;
-    q.r2 = r2;
-    q.first = it == 0;
-    if (fused) {
-      apply(q);
-    } else {
-      hipLaunchKernelGGL(mr_gemv_rows, dim3((unsigned)(Ns + 2)), dim3(512), 0, st, Ns, Np, O,
-                         o_dtype, ldo, q, rtol, inner, sc);
+  if (Np <= kNarrowNp) {
+    const int n = (int)Np;
+    MrVecs q{};
+    q.m = m;
+    q.x = x;
+    for (int it = 0; it < maxiter; ++it) {
+      q.r1 = r1;
+      q.r2 = r2;
+      q.first = it == 0;
+      hipLaunchKernelGGL(mr_rows, dim3((unsigned)((Ns + 3) / 4 + 2)), dim3(1024), 0, st, Ns, n,
+                         nbd, O, o_dtype, ldo, q, rtol, inner, sc);
       hipLaunchKernelGGL(mr_colsum_partial, dim3(gn, kRowChunks), dim3(256), 0, st, Ns, Np, O,
                          o_dtype, ldo, rows, (const double *)inner, (const double *)nullptr,
-                         partial, partial2, done);
+                         partial, partial2, (const double *)(sc + S_STOP));
+      hipLaunchKernelGGL(mr_form_y_narrow, dim3((unsigned)((Np + 63) / 64)), dim3(64), 0, st, n,
+                         partial, 1.0 / (double)Ns, m, r1, r2, diag_shift, y, sc);
+      hipLaunchKernelGGL(mr_finish, dim3(1), dim3(1024), 0, st, n, nbd, r2, y, sc);
+      VMCX_LAUNCHED();
+      // r1 <- r2 <- y; the x update of this iteration (with its v = r2 / beta, then r1 /
+      // oldb) runs in the next one's first launch: w1 <- w2 <- w (buffers rotate on the
+      // host; once the device flag is set nothing reads them again)
+      double *t = r1;
+      r1 = r2;
+      r2 = y;
+      y = t;
+      q.w1 = w1;
+      q.w2 = w2;
+      q.w = wn;
+      t = w1;
+      w1 = w2;
+      w2 = wn;
+      wn = t;
     }
-    hipLaunchKernelGGL(mr_form_y, dim3(yb), dim3(1024), 0, st, Np, chunks, partial,
-                       1.0 / (double)Ns, m, r1, r2, diag_shift, y, dotp, sc);
-    hipLaunchKernelGGL(mr_finish, dim3(1), dim3(1024), 0, st, Np, (int64_t)yb, dotp, r2, y, sc);
-    VMCX_LAUNCHED();
-    // r1 <- r2 <- y; the x update of this iteration (with its v = r2 / beta, then r1 /
-    // oldb) runs in the next one's first launch: w1 <- w2 <- w (buffers rotate on the
-    // host; once the device flag is set nothing reads them again)
-    double *t = r1;
-    r1 = r2;
-    r2 = y;
-    y = t;
-    q.w1 = w1;
-    q.w2 = w2;
-    q.w = wn;
-    t = w1;
-    w1 = w2;
-    w2 = wn;
-    wn = t;
-  }
-  if (maxiter > 0) {
-    q.r1 = r1;
-    q.r2 = r2;
-    hipLaunchKernelGGL(mr_last_update, dim3(1), dim3(512), 0, st, Np, q, rtol, sc);
+    if (maxiter > 0) {
+      q.r1 = r1;
+      q.r2 = r2;
+      hipLaunchKernelGGL(mr_last_update, dim3(1), dim3(1024), 0, st, n, nbd, q, rtol, sc);
+    }
+  } else {
+    // v and S v: the second set of chunk sums is free after Obar and g
+    double *v = partial2, *Sx = partial2 + Np;
+    for (int it = 0; it < maxiter; ++it) {
+      hipLaunchKernelGGL(mr_scale_v, dim3(gn), dim3(256), 0, st, Np, r2, v, sc);
+      // S v without S: O v, then O^T (O v) / Ns
+      hipLaunchKernelGGL(mr_gemv_rows, dim3((unsigned)Ns), dim3(256), 0, st, Np, O, o_dtype, ldo,
+                         v, inner, sc);
+      hipLaunchKernelGGL(mr_colsum_partial, dim3(gn, kRowChunks), dim3(256), 0, st, Ns, Np, O,
+                         o_dtype, ldo, rows, (const double *)inner, (const double *)nullptr,
+                         partial, (double *)nullptr, done);
+      hipLaunchKernelGGL(mr_colsum_final, dim3(gn), dim3(256), 0, st, Np, partial,
+                         1.0 / (double)Ns, Sx, done);
+      dot(m, v, S_MV, done);
+      hipLaunchKernelGGL(mr_form_y, dim3(gn), dim3(256), 0, st, Np, Sx, m, v, r1, diag_shift, y,
+                         sc);
+      dot(v, y, S_ALFA, done);
+      hipLaunchKernelGGL(mr_orth_y, dim3(gn), dim3(256), 0, st, Np, r2, y, sc);
+      dot(y, y, S_BETA2, done);
+      hipLaunchKernelGGL(mr_rotate, dim3(1), dim3(1), 0, st, sc);
+      hipLaunchKernelGGL(mr_update_x, dim3(gn), dim3(256), 0, st, Np, v, w1, w2, wn, x, sc);
+      dot(x, x, S_YNORM2, done);
+      hipLaunchKernelGGL(mr_check, dim3(1), dim3(1), 0, st, rtol, sc);
+      VMCX_LAUNCHED();
+      // r1 <- r2 <- y ; w1 <- w2 <- w (buffers rotate on the host; once the
+      // device flag is set nothing reads them again)
+      double *t = r1;
+      r1 = r2;
+      r2 = y;
+      y = t;
+      t = w1;
+      w1 = w2;
+      w2 = wn;
+      wn = t;
+    }
   }
   hipLaunchKernelGGL(mr_stats, dim3(1), dim3(1), 0, st, sc, stats, info);
   VMCX_LAUNCHED();

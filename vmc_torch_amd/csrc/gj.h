@@ -258,8 +258,9 @@ struct LuStep<NFP, NFP, T> {
 // Bound by the vector instructions and the dependent chain of the 64 pivot searches.  A
 // step of the unblocked elimination updates up to 63 entries of a lane with up to 63
 // broadcasts, and its 64 unrolled steps exceed the instruction cache; here it is 15 and 15,
-// and the four panels share one code.  Measured: one wave's FP64 determinant, with its loads,
-// in nnbf_accept_kernel 64 -> 38 us.
+// with 120 broadcasts and updates a panel for the pivot rows, and the four panels share one
+// code.  Measured: one wave's FP64 determinant, with its loads, in nnbf_accept_kernel 41 us
+// (unblocked 64); 8192 of 64 x 64 in refresh_kernel without A^-1 195 us (203).
 // multiplier a / piv: FP32 by the hardware reciprocal (1 ulp), FP64 by the
 // correctly rounded division
 __device__ __forceinline__ float lu_mult(float a, float piv) {
@@ -340,63 +341,64 @@ struct LuTile<double> {
 };
 
 // Step P of a panel x[16] (lane = row): pivot by DPP arg-max, then every row takes f times
-// the pivot row away.  x[P] ends as f, and the multipliers of earlier steps are updated with
-// the rest, so that after the panel x holds the W of "row -= sum_p W[row][p] pivot row p of
-// the matrix before the panel".  The pivot row's half that holds P is broadcast by readlane,
-// the other half through LDS.
+// the pivot row's entries right of P away.  x[P] ends as f, lanes[P] as the pivot's lane.  The
+// pivot row's entries of the half that holds P are broadcast by readlane, those of the half
+// right of it through LDS.
 template <int P, typename T>
 struct LuPanel {
   static __device__ __forceinline__ void run(T (&x)[16], int col, T &pivs, uint64_t &used,
-                                             int &parity, int &step, T *buf) {
-    typedef LuVec<T> V;
+                                             int &parity, int &step, int (&lanes)[16], T *buf) {
     const T mag = fabs(x[P]);
     const float fm = (mag <= lu_big<T>()) ? (float)mag : 0.0f;
     const uint32_t key = (__float_as_uint(fm) & ~63u) | (uint32_t)(63 - col);
     const int q = 63 - (int)(lu_wave_max(key) & 63u);
     const bool mine = col == q;
-    constexpr int near = P & 8, far = 8 - near;
-    if (mine) {
+    constexpr int near = P & 8;
+    if (near == 0 && mine) {
 #pragma unroll
-      for (int j = 0; j < 8; j += V::n)
-        *reinterpret_cast<typename V::t *>(buf + j) = V::make(&x[far + j]);
+      for (int j = 0; j < 8; j += 2)
+        *reinterpret_cast<double2 *>(buf + j) = make_double2(x[8 + j], x[9 + j]);
     }
     const T piv = lu_bcast(x[P], q);
     pivs = mine ? piv : pivs;
     step = mine ? P : step;
+    lanes[P] = q;
     const T f = mine ? T(1) : lu_mult(x[P], piv);
     T r[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (near + j != P) r[j] = lu_bcast(x[near + j], q);
+      if (near + j > P) r[j] = lu_bcast(x[near + j], q);
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (near + j != P) x[near + j] = fma(-f, r[j], x[near + j]);
+      if (near + j > P) x[near + j] = fma(-f, r[j], x[near + j]);
     x[P] = f;
-    wave_lds_fence();
+    if (near == 0) {
+      wave_lds_fence();
 #pragma unroll
-    for (int j = 0; j < 8; j += V::n) {
-      const typename V::t v = *reinterpret_cast<const typename V::t *>(buf + j);
-      x[far + j] = fma(-f, v.x, x[far + j]);
-      x[far + j + 1] = fma(-f, v.y, x[far + j + 1]);
-      if constexpr (V::n == 4) {
-        x[far + j + 2] = fma(-f, v.z, x[far + j + 2]);
-        x[far + j + 3] = fma(-f, v.w, x[far + j + 3]);
+      for (int j = 0; j < 8; j += 2) {
+        const double2 v = *reinterpret_cast<const double2 *>(buf + j);
+        x[8 + j] = fma(-f, v.x, x[8 + j]);
+        x[9 + j] = fma(-f, v.y, x[9 + j]);
       }
+      wave_lds_fence();
     }
-    wave_lds_fence();
     // row exchanges: lanes chosen earlier with a higher index than q
     parity += __popcll(used & ~((2ull << q) - 1ull));
     used |= 1ull << q;
-    LuPanel<P + 1, T>::run(x, col, pivs, used, parity, step, buf);
+    LuPanel<P + 1, T>::run(x, col, pivs, used, parity, step, lanes, buf);
   }
 };
 
 template <typename T>
 struct LuPanel<16, T> {
-  static __device__ __forceinline__ void run(T (&)[16], int, T &, uint64_t &, int &, int &, T *) {}
+  static __device__ __forceinline__ void run(T (&)[16], int, T &, uint64_t &, int &, int &,
+                                             int (&)[16], T *) {}
 };
 
-// all four panels; the columns to the right of a panel are updated on the matrix cores
+// All four panels.  The columns to the right of a panel: its 16 pivot rows are carried through
+// the panel's steps first (lane = column, three tiles of 16 columns at once), then the other
+// rows take their multiples away on the matrix cores.  Every entry takes the same
+// multiply-adds in the same order as unblocked, step by step, so the result is the same.
 template <typename T>
 __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64_t &used,
                                             int &parity, T *buf) {
@@ -420,33 +422,60 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
   }
 #pragma unroll 1
   for (int k = 0; k < 4; ++k) {
-    int step = -1;
-    LuPanel<0, T>::run(pan, col, pivs, used, parity, step, buf);
+    int step = -1, lanes[16];
+    LuPanel<0, T>::run(pan, col, pivs, used, parity, step, lanes, buf);
     if (k == 3) break;
-    v4 W[4];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) pan[j] = -pan[j];
-    L::to_blocks(pan, W);
     uint32_t rk[4] = {(uint32_t)step, (uint32_t)step, (uint32_t)step, (uint32_t)step};
     lu_swap4(rk[0], rk[1], rk[2], rk[3]);   // step of row 16 g + x
+    T u[16];
+#pragma unroll
+    for (int p = 0; p < 16; ++p) u[p] = T(0);
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       if (t < 3 - k) {
-        // the panel's pivot rows of the tile, as the left operand
+        // the panel's pivot rows of tile t: from here on they are zero
 #pragma unroll
         for (int g = 0; g < 4; ++g)
           if ((int)rk[g] >= 0) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) buf[(int)rk[g] * LD + L::column(c, r)] = tile[t][g][r];
+            for (int r = 0; r < 4; ++r) {
+              buf[(int)rk[g] * LD + L::column(c, r)] = tile[t][g][r];
+              tile[t][g][r] = T(0);
+            }
           }
         wave_lds_fence();
-        T u[4];
+        if (c == t) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) u[r] = buf[L::column(c, r) * LD + x];
+          for (int p = 0; p < 16; ++p) u[p] = buf[p * LD + x];
+        }
+        wave_lds_fence();
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 15; ++q) {
+#pragma unroll
+      for (int p = q + 1; p < 16; ++p) u[p] = fma(-lu_bcast(pan[q], lanes[p]), u[q], u[p]);
+      __builtin_amdgcn_sched_barrier(0);   // (all readlanes at once overflow the registers)
+    }
+    v4 W[4];
+#pragma unroll
+    for (int j = 0; j < 16; ++j) pan[j] = step >= 0 ? T(0) : -pan[j];
+    L::to_blocks(pan, W);
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+      if (t < 3 - k) {
+        if (c == t) {
+#pragma unroll
+          for (int p = 0; p < 16; ++p) buf[p * LD + x] = u[p];
+        }
+        wave_lds_fence();
+        T v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = buf[L::column(c, r) * LD + x];
 #pragma unroll
         for (int r = 0; r < 4; ++r)
 #pragma unroll
-          for (int g = 0; g < 4; ++g) tile[t][g] = L::mfma(u[r], W[g][r], tile[t][g]);
+          for (int g = 0; g < 4; ++g) tile[t][g] = L::mfma(v[r], W[g][r], tile[t][g]);
         wave_lds_fence();
       }
     }
@@ -459,10 +488,7 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
   }
 }
 
-// FP32: unblocked.  The panels' update, formed from the pivot rows as they were before the
-// panel, loses a little to cancellation (median error of ln|det| 6 %, 99th percentile 10 to
-// 20 % above this one, over 8192 configurations at n_f = 36 to 64); in FP64 the two agree
-// (medians 7.4e-15 and 7.6e-15 against extended precision at n_f = 64).
+// FP32: unblocked.
 // The pivot row reaches the other lanes by readlane (its head: two vector instructions per
 // entry with the update) and through the wave's LDS buffer (its tail, 4/6: one), the split
 // that keeps both pipes busy.

@@ -1159,7 +1159,7 @@ __global__ void masked_rows_kernel(int64_t B, int64_t row_words, const uint8_t *
 // proposal on the next edge (if `more`).  The commit's columns of W1 are read from the
 // transposed weights, eight of a lane's units in flight.
 // Bound by the latency of one elimination (lu_logdet).  Measured, FP64: 6x6 (n_f = 32), 4096
-// walkers 38 us; 8x8 (n_f = 64), 1000 walkers 38 us (45.8 and 64 with a branch per row of the
+// walkers 38 us; 8x8 (n_f = 64), 1000 walkers 41 us (45.8 and 64 with a branch per row of the
 // matrix and the unblocked elimination).
 template <int NFP, typename TW>
 __global__ void __launch_bounds__(256)

@@ -533,14 +533,18 @@ __device__ __forceinline__ int p64_v(int D, int odd, int t) {
 // Table of column operands, one workgroup per (combination, half, column):
 // tab[((y 2 + half) 64 + q) P64_CELL + ((t 2 + r / 2) 64 + lane) 2 + r % 2], q = (8 q0 + q1)
 // of the half's rows (2 state + parity each; q0 alone with one row).  First of several
-// columns (dimension 1 on the left): register 0 of pair 0, [a'][v] (k = v); last column
-// (dimension 1 on the right): pair 0, [a][v].
+// columns (dimension 1 on the left): register 0 of pair 0, [a'][v] (k = v), scaled by a power
+// of two to a largest entry of about 1 (the environment is first scaled after the second
+// column: eight slices' product otherwise), its exponent in entry 1; last column (dimension 1
+// on the right): pair 0, [a][v].
 __global__ void __launch_bounds__(256) peps_col_table_kernel(PepsArgs A, double *tab) {
   const PepsGeo &g = A.g;
   const int q = blockIdx.x, half = blockIdx.y, y = blockIdx.z, D = g.D, tid = threadIdx.x;
   const int x0 = half ? g.tr : 0, nr = half ? g.Lx - g.tr : g.tr;
   if (nr == 1 && q >= 8) return;
   __shared__ double sl[2][SLICE];
+  __shared__ int mex;
+  if (tid == 0) mex = 0;
   const int q0 = nr == 2 ? q >> 3 : q, q1 = nr == 2 ? q & 7 : 0;
   int off = 0, par = 0;
   for (int s = 0; s < g.N; ++s) {
@@ -592,7 +596,17 @@ __global__ void __launch_bounds__(256) peps_col_table_kernel(PepsArgs A, double 
       if (a < da && li < da2) v = entry(a, p64_v(D, par ^ pa ^ pb, t), li);
     }
     cell[idx] = v;
+    if (idx < 128 && y == 0) {
+      int e = (__double2hiint(v) >> 20) & 0x7FF;
+      for (int o = 32; o > 0; o >>= 1) e = max(e, __shfl_xor(e, o, 64));
+      if ((tid & 63) == 0) atomicMax(&mex, e);
+    }
   }
+  if (y > 0 || g.Ly == 1) return;
+  __syncthreads();
+  // all zero, infinite or NaN: left alone
+  const int ex = mex > 0 && mex < 0x7FF ? mex - 1023 : 0;
+  if (tid < 128) cell[tid] = tid & 1 ? (double)ex : ldexp(cell[tid], -ex);
 }
 
 // the wave's largest exponent field of four doubles per lane
@@ -653,10 +667,12 @@ __device__ __forceinline__ void peps_amp_wave(const PepsGeo &g, const double *__
   };
   p64d4 env = {lane == 0 ? 1.0 : 0.0, 0.0, 0.0, 0.0};
   int esc = 0, par = 0;
+  double ex0 = 0.0;   // the first column's exponent
   Ops cur, nxt;
   int y = 0;
   if (Ly > 1) {
     const double ft = cell(0, 0)[lane].x, fb = cell(0, 1)[lane].x;
+    ex0 = cell(0, 0)[0].y + cell(0, 1)[0].y;
     load(1, cur);
     const p64d4 z = {0.0, 0.0, 0.0, 0.0};
     env = __builtin_amdgcn_mfma_f64_16x16x4f64(ft, fb, z, 0, 0, 0);
@@ -717,7 +733,7 @@ __device__ __forceinline__ void peps_amp_wave(const PepsGeo &g, const double *__
     logabs = lo;
   } else {
     sign = v > 0.0 ? 1.0 : -1.0;
-    logabs = fmax(log(fabs(v)) + esc * 0.693147180559945309417, lo);
+    logabs = fmax(log(fabs(v)) + (esc + ex0) * 0.693147180559945309417, lo);
   }
 }
 

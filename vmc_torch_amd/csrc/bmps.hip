@@ -52,13 +52,23 @@ constexpr int BMAX_SWEEPS = 30;
 // this floor are not rotated away (singular values below ~1e-9 of the
 // largest, which move an amplitude by about that much relative)
 constexpr double BM_ROT_FLOOR = 1e-18;
-// the pivoted Cholesky stops when the largest remaining diagonal entry is below this:
-// graded states (bond entries that fall off by 10 per index) need the small singular
-// values, which the factor and one-sided Jacobi keep to relative accuracy.  Against the
-// QR / SVD truncation, median relative error of an amplitude of such a 6x6 D = 4 chi = 8
-// state: 3e-8 with a floor of 4.4e-16, 3e-10 with 1e-18, 6e-11 with 1e-24 and below
-// (7e-10 with two-sided Jacobi); the floors cost the same time from 1e-18 on
+// A pivot of the Cholesky factor must exceed BM_PIVOT_FLOOR (of the block's largest diagonal
+// entry) and BM_PIVOT_NOISE of its own row's diagonal entry at the start.
+// The second: a remainder d below the rounding of its row's entries (a few ulp of the
+// diagonal) is noise, and noise^2 / d, which may be of any size where d happens to be small,
+// would enter the factor.  With d above one ulp LL^T stays within 1e-13 of the block, in units
+// of sqrt(A_ii A_jj) (NumPy, 2e5 16 x 16 blocks of rank 8: worst 3e-10 without, 1e-13 with
+// half an ulp, 3e-14 with two), and no noise column is larger than a direction of
+// eigenvalue 256 ulp, which it could push out of the chi kept ones: a D = 2 state written with
+// D = 4, 6x6 chi = 8, 32768 amplitudes: 99.9 % within 3e-10, worst 8e-8; without 2e-9 and 1e-5
+// (two-sided Jacobi 1e-9 and 1e-5).
+// Neither may be larger: graded states (bond entries that fall off by 10 per index) need the
+// small singular values, which the factor and one-sided Jacobi keep to relative accuracy, and
+// their rows are graded likewise.  Against the QR / SVD truncation, median relative error of
+// an amplitude, 6x6 D = 4 chi = 8 and 6x6 D = 2 chi = 6: 7e-11 and 2.6e-12 (two-sided Jacobi
+// 8e-10 and 6e-12; BM_PIVOT_NOISE of 16 ulp 8e-11 and 9e-12; a floor of 4.4e-16 3e-8).
 constexpr double BM_PIVOT_FLOOR = 1e-30;
+constexpr double BM_PIVOT_NOISE = 2.220446049250313e-16;
 // int64 header words per boundary buffer: [0] log scale (double bits),
 // [1 .. Ly+1] bond dimensions, [Ly+2 .. 2Ly+2] bond parity masks
 constexpr int BHDR = 40;
@@ -290,7 +300,7 @@ __device__ __forceinline__ double bm_rsqrt(double x) {
 // workgroups on a CU: 80 k cycles; 198 k on the columns of the block itself, and 1754 us
 // per launch of 2048 workgroups with two-sided Jacobi in LDS against 1020 us with this.
 // Columns are orthogonal to 4e-15 of their own norms; what the
-// factorisation leaves out (BM_PIVOT_FLOOR) comes out as zero vectors.
+// factorisation leaves out (BM_PIVOT_FLOOR, BM_PIVOT_NOISE) comes out as zero vectors.
 // row: LDS scratch of 4 RPL doubles per block.
 // Output, compacted: columns off .. off + m of T (rows off .. off + m) and lam; the
 // caller has zeroed both, or (CLEAR, JB = 3, off = 0, 16 x ld each) they are zeroed here
@@ -318,11 +328,13 @@ __device__ __forceinline__ void bm_jacobi_wave(const double *R, int ld, int off,
     }
     double dt = c0 < m ? R[(off + c0) * (ld + 1)] : 0.0;
     double db = c1 < m ? R[(off + c1) * (ld + 1)] : 0.0;
+    const double ft = fmax(BM_PIVOT_FLOOR, BM_PIVOT_NOISE * dt);
+    const double fb = fmax(BM_PIVOT_FLOOR, BM_PIVOT_NOISE * db);
     constexpr unsigned IM = 2 * NJ - 1;
     for (int step = 0; step < mmax; ++step) {
       // largest remaining diagonal entry (to FP32 precision, the column in the low bits)
-      const unsigned kt = dt > BM_PIVOT_FLOOR ? (__float_as_uint((float)dt) & ~IM) | c0 : 0u;
-      const unsigned kb = db > BM_PIVOT_FLOOR ? (__float_as_uint((float)db) & ~IM) | c1 : 0u;
+      const unsigned kt = dt > ft ? (__float_as_uint((float)dt) & ~IM) | c0 : 0u;
+      const unsigned kb = db > fb ? (__float_as_uint((float)db) & ~IM) | c1 : 0u;
       unsigned key = kt > kb ? kt : kb;
       key = max(key, (unsigned)bm_xor32<1>((int)key));
       key = max(key, (unsigned)bm_xor32<2>((int)key));

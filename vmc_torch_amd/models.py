@@ -591,11 +591,13 @@ class fPEPS_Model_GPU(WavefunctionModel_GPU):
 
     def _sync(self):
         """The struct the kernels read: it points to the parameters
-        themselves, so only a moved tensor needs a new one."""
+        themselves, so only a moved tensor or another option needs a new one."""
         for p in self.params:
             if not p.data.is_contiguous():
                 p.data = p.data.contiguous()
-        at = tuple(p.data_ptr() for p in self.params) + (self.dense_map.data_ptr(),)
+        at = tuple(p.data_ptr() for p in self.params) + (
+            self.dense_map.data_ptr(), self.eta, self.mode, self.act_name, self.amp, self.chi,
+            self.bmps_cache)
         if self._struct_obj is None or self._struct_at != at:
             self._struct_obj = kernels.peps_struct(
                 self.Lx, self.Ly, self.D, self.dense_map, self.params[0].data,
@@ -874,12 +876,10 @@ class fPEPS_Model_reuse_GPU(fPEPS_Model_GPU):
             return fn(self, *args, **kwargs)
         keep = self.bmps_cache
         self.bmps_cache = False   # every row recontracted
-        self._struct_obj = None
         try:
             return fn(self, *args, **kwargs)
         finally:
             self.bmps_cache = keep
-            self._struct_obj = None
 
     def mcmc_sweep_full(self, *args, **kwargs):
         return self._full(fPEPS_Model_GPU.mcmc_sweep, *args, **kwargs)
@@ -940,8 +940,16 @@ class NNfTNS_Model_GPU(fPEPS_Model_GPU):
                          chunk=chunk, _nn=nnp, act=activation, eta=nn_eta,
                          _mode=self.CORRECTIONS[correction], amp=amp)
         self.hidden = hidden_dim
-        self.nn_eta = float(nn_eta)
         self.correction = correction
+
+    # the scale of the correction: eta under the reference's name
+    @property
+    def nn_eta(self):
+        return self.eta
+
+    @nn_eta.setter
+    def nn_eta(self, value):
+        self.eta = float(value)
 
     def _nn_dict(self):
         names = ["W1", "b1", "W2", "b2", "Wo", "bo"]

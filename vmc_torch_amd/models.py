@@ -146,7 +146,7 @@ class SlaterDeterminant_GPU(WavefunctionModel_GPU):
             self._m64 = torch.empty(M.shape, dtype=torch.float64, device=M.device) \
                 if self.fp32 else None
             force = True
-        kernels.slater_mark_params(M, self._built_from, self._m64, state, force)
+        kernels.slater_mark_params(M.contiguous(), self._built_from, self._m64, state, force)
 
     def _m_f64(self):
         """M in FP64 for the exact refresh (M itself in the plain form; the

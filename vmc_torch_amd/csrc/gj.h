@@ -268,23 +268,6 @@ __device__ __forceinline__ float lu_mult(float a, float piv) {
 }
 __device__ __forceinline__ double lu_mult(double a, double piv) { return a / piv; }
 
-// 16-byte vectors of the LDS part
-template <typename T>
-struct LuVec;
-template <>
-struct LuVec<float> {
-  typedef float4 t;
-  static constexpr int n = 4, tail6 = 4;
-  static __device__ __forceinline__ t make(const float *x) {
-    return make_float4(x[0], x[1], x[2], x[3]);
-  }
-};
-template <>
-struct LuVec<double> {
-  typedef double2 t;
-  static constexpr int n = 2, tail6 = 3;
-  static __device__ __forceinline__ t make(const double *x) { return make_double2(x[0], x[1]); }
-};
 // Exchange of register blocks and lane groups: reg[c] of lane group g <-> reg[g] of lane
 // group c (groups of 16 lanes, four registers).
 __device__ __forceinline__ void lu_swap4(uint32_t &r0, uint32_t &r1, uint32_t &r2, uint32_t &r3) {
@@ -313,10 +296,7 @@ __device__ __forceinline__ void lu_swap4(double &a, double &b, double &c, double
 // 64 x 16 tile of the matrix as the matrix-core result of its transpose (row block g of 16:
 // lane l holds row 16 g + l % 16 and four columns), and back: between it and "lane = row,
 // register = column" the lane group trades places with one digit of the column.
-template <typename T>
-struct LuTile;
-template <>
-struct LuTile<double> {
+struct LuTile {
   typedef double v4 __attribute__((ext_vector_type(4)));
   static __device__ __forceinline__ int column(int c, int r) { return 4 * r + c; }
   static __device__ __forceinline__ v4 mfma(double a, double b, v4 x) {
@@ -344,12 +324,12 @@ struct LuTile<double> {
 // the pivot row's entries right of P away.  x[P] ends as f, lanes[P] as the pivot's lane.  The
 // pivot row's entries of the half that holds P are broadcast by readlane, those of the half
 // right of it through LDS.
-template <int P, typename T>
+template <int P>
 struct LuPanel {
-  static __device__ __forceinline__ void run(T (&x)[16], int col, T &pivs, uint64_t &used,
-                                             int &parity, int &step, int (&lanes)[16], T *buf) {
-    const T mag = fabs(x[P]);
-    const float fm = (mag <= lu_big<T>()) ? (float)mag : 0.0f;
+  static __device__ __forceinline__ void run(double (&x)[16], int col, double &pivs, uint64_t &used,
+                                             int &parity, int &step, int (&lanes)[16], double *buf) {
+    const double mag = fabs(x[P]);
+    const float fm = (mag <= lu_big<double>()) ? (float)mag : 0.0f;
     const uint32_t key = (__float_as_uint(fm) & ~63u) | (uint32_t)(63 - col);
     const int q = 63 - (int)(lu_wave_max(key) & 63u);
     const bool mine = col == q;
@@ -359,12 +339,12 @@ struct LuPanel {
       for (int j = 0; j < 8; j += 2)
         *reinterpret_cast<double2 *>(buf + j) = make_double2(x[8 + j], x[9 + j]);
     }
-    const T piv = lu_bcast(x[P], q);
+    const double piv = lu_bcast(x[P], q);
     pivs = mine ? piv : pivs;
     step = mine ? P : step;
     lanes[P] = q;
-    const T f = mine ? T(1) : lu_mult(x[P], piv);
-    T r[8];
+    const double f = mine ? 1.0 : lu_mult(x[P], piv);
+    double r[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j)
       if (near + j > P) r[j] = lu_bcast(x[near + j], q);
@@ -385,32 +365,31 @@ struct LuPanel {
     // row exchanges: lanes chosen earlier with a higher index than q
     parity += __popcll(used & ~((2ull << q) - 1ull));
     used |= 1ull << q;
-    LuPanel<P + 1, T>::run(x, col, pivs, used, parity, step, lanes, buf);
+    LuPanel<P + 1>::run(x, col, pivs, used, parity, step, lanes, buf);
   }
 };
 
-template <typename T>
-struct LuPanel<16, T> {
-  static __device__ __forceinline__ void run(T (&)[16], int, T &, uint64_t &, int &, int &,
-                                             int (&)[16], T *) {}
+template <>
+struct LuPanel<16> {
+  static __device__ __forceinline__ void run(double (&)[16], int, double &, uint64_t &, int &, int &,
+                                             int (&)[16], double *) {}
 };
 
 // All four panels.  The columns to the right of a panel: its 16 pivot rows are carried through
 // the panel's steps first (lane = column, three tiles of 16 columns at once), then the other
 // rows take their multiples away on the matrix cores.  Every entry takes the same
 // multiply-adds in the same order as unblocked, step by step, so the result is the same.
-template <typename T>
-__device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64_t &used,
-                                            int &parity, T *buf) {
-  typedef LuTile<T> L;
-  typedef typename L::v4 v4;
+__device__ __forceinline__ void lu64_panels(double (&a)[64], int col, double &pivs, uint64_t &used,
+                                            int &parity, double *buf) {
+  typedef LuTile L;
+  typedef L::v4 v4;
   constexpr int LD = 20;      // LDS row of a tile of 16
   const int c = col >> 4, x = col & 15;
-  T pan[16];
+  double pan[16];
   v4 tile[3][4];
 #pragma unroll
   for (int t = 0; t < 4; ++t) {
-    T y[16];
+    double y[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) y[j] = a[16 * t + j];
     if (t == 0) {
@@ -423,13 +402,13 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
 #pragma unroll 1
   for (int k = 0; k < 4; ++k) {
     int step = -1, lanes[16];
-    LuPanel<0, T>::run(pan, col, pivs, used, parity, step, lanes, buf);
+    LuPanel<0>::run(pan, col, pivs, used, parity, step, lanes, buf);
     if (k == 3) break;
     uint32_t rk[4] = {(uint32_t)step, (uint32_t)step, (uint32_t)step, (uint32_t)step};
     lu_swap4(rk[0], rk[1], rk[2], rk[3]);   // step of row 16 g + x
-    T u[16];
+    double u[16];
 #pragma unroll
-    for (int p = 0; p < 16; ++p) u[p] = T(0);
+    for (int p = 0; p < 16; ++p) u[p] = 0.0;
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
       if (t < 3 - k) {
@@ -440,7 +419,7 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               buf[(int)rk[g] * LD + L::column(c, r)] = tile[t][g][r];
-              tile[t][g][r] = T(0);
+              tile[t][g][r] = 0.0;
             }
           }
         wave_lds_fence();
@@ -459,7 +438,7 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
     }
     v4 W[4];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) pan[j] = step >= 0 ? T(0) : -pan[j];
+    for (int j = 0; j < 16; ++j) pan[j] = step >= 0 ? 0.0 : -pan[j];
     L::to_blocks(pan, W);
 #pragma unroll
     for (int t = 0; t < 3; ++t) {
@@ -469,7 +448,7 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
           for (int p = 0; p < 16; ++p) buf[p * LD + x] = u[p];
         }
         wave_lds_fence();
-        T v[4];
+        double v[4];
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = buf[L::column(c, r) * LD + x];
 #pragma unroll
@@ -492,38 +471,37 @@ __device__ __forceinline__ void lu64_panels(T (&a)[64], int col, T &pivs, uint64
 // The pivot row reaches the other lanes by readlane (its head: two vector instructions per
 // entry with the update) and through the wave's LDS buffer (its tail, 4/6: one), the split
 // that keeps both pipes busy.
-template <int P, typename T>
+template <int P>
 struct LuStep64 {
-  static __device__ __forceinline__ void run(T (&a)[64], int col, T &pivs, uint64_t &used,
-                                             int &parity, T *buf) {
+  static __device__ __forceinline__ void run(float (&a)[64], int col, float &pivs, uint64_t &used,
+                                             int &parity, float *buf) {
     // pivot key: |a| rounded to float with its 6 low mantissa bits replaced
     // by 63 - lane (largest magnitude to 2^-17, then the lowest lane); NaN /
     // Inf rank as 0
-    const T mag = fabs(a[P]);
-    const float fm = (mag <= lu_big<T>()) ? (float)mag : 0.0f;
+    const float mag = fabs(a[P]);
+    const float fm = (mag <= lu_big<float>()) ? (float)mag : 0.0f;
     const uint32_t key = (__float_as_uint(fm) & ~63u) | (uint32_t)(63 - col);
     const int q = 63 - (int)(lu_wave_max(key) & 63u);
-    const T piv = lu_bcast(a[P], q);
+    const float piv = lu_bcast(a[P], q);
     const bool mine = col == q;
     pivs = mine ? piv : pivs;
     if (P + 1 < 64) {
-      const T f = mine ? T(1) : lu_mult(a[P], piv);
-      typedef LuVec<T> V;
+      const float f = mine ? 1.0f : lu_mult(a[P], piv);
       // entries [P + 1, js) by readlane, [js, 64) through LDS (js aligned)
-      constexpr int n_tail = ((63 - P) * V::tail6) / 6;
-      constexpr int js0 = (64 - n_tail + V::n - 1) & ~(V::n - 1);
-      constexpr int js = js0 < P + 1 ? ((P + 1 + V::n - 1) & ~(V::n - 1)) : js0;
+      constexpr int n_tail = ((63 - P) * 4) / 6;
+      constexpr int js0 = (64 - n_tail + 3) & ~3;
+      constexpr int js = js0 < P + 1 ? ((P + 1 + 3) & ~3) : js0;
       if (js < 64 && mine) {
 #pragma unroll
-        for (int j = js; j < 64; j += V::n)
-          *reinterpret_cast<typename V::t *>(buf + j) = V::make(&a[j]);
+        for (int j = js; j < 64; j += 4)
+          *reinterpret_cast<float4 *>(buf + j) = make_float4(a[j], a[j + 1], a[j + 2], a[j + 3]);
       }
       // blocks of 8 readlane entries kept apart by scheduling barriers, so
       // that the readlanes of one block are consumed before the next block's
       // are issued (hoisting all of them overflows the scalar registers)
 #pragma unroll
       for (int j0 = P + 1; j0 < js && j0 < 64; j0 += 8) {
-        T r[8];
+        float r[8];
 #pragma unroll
         for (int k = 0; k < 8; ++k)
           if (j0 + k < js && j0 + k < 64) r[k] = lu_bcast(a[j0 + k], q);
@@ -535,14 +513,12 @@ struct LuStep64 {
       if (js < 64) {
         wave_lds_fence();
 #pragma unroll
-        for (int j = js; j < 64; j += V::n) {
-          const typename V::t v = *reinterpret_cast<const typename V::t *>(buf + j);
+        for (int j = js; j < 64; j += 4) {
+          const float4 v = *reinterpret_cast<const float4 *>(buf + j);
           a[j] = fma(-f, v.x, a[j]);
           a[j + 1] = fma(-f, v.y, a[j + 1]);
-          if constexpr (V::n == 4) {
-            a[j + 2] = fma(-f, v.z, a[j + 2]);
-            a[j + 3] = fma(-f, v.w, a[j + 3]);
-          }
+          a[j + 2] = fma(-f, v.z, a[j + 2]);
+          a[j + 3] = fma(-f, v.w, a[j + 3]);
         }
         // the buffer is rewritten by the next step's pivot lane
         wave_lds_fence();
@@ -551,13 +527,13 @@ struct LuStep64 {
     // row exchanges: lanes chosen earlier with a higher index than q
     parity += __popcll(used & ~((2ull << q) - 1ull));
     used |= 1ull << q;
-    LuStep64<P + 1, T>::run(a, col, pivs, used, parity, buf);
+    LuStep64<P + 1>::run(a, col, pivs, used, parity, buf);
   }
 };
 
-template <typename T>
-struct LuStep64<64, T> {
-  static __device__ __forceinline__ void run(T (&)[64], int, T &, uint64_t &, int &, T *) {}
+template <>
+struct LuStep64<64> {
+  static __device__ __forceinline__ void run(float (&)[64], int, float &, uint64_t &, int &, float *) {}
 };
 
 // sign and log|det| from the 64 pivots (lane l: the pivot taken from lane
@@ -585,10 +561,10 @@ __device__ __forceinline__ GJResult lu_logdet(T (&a)[NFP], int col, int gbase, T
     uint64_t used = 0ull;
     int parity = 0;
     if constexpr (sizeof(T) == 4) {
-      LuStep64<0, T>::run(a, col, pivs, used, parity, prow);
+      LuStep64<0>::run(a, col, pivs, used, parity, prow);
     } else {
       __shared__ __align__(16) T buf[8][16 * 20];   // (callers: at most eight waves)
-      lu64_panels<T>(a, col, pivs, used, parity, buf[threadIdx.x >> 6]);
+      lu64_panels(a, col, pivs, used, parity, buf[threadIdx.x >> 6]);
     }
     GJResult r{0.0, 0, false, -1};
     lu64_finish(pivs, used, parity, r.logdet, r.parity, r.singular);

@@ -18,13 +18,14 @@
 // Per iteration, up to kNarrowNp parameters, four launches:
 //   mr_rows        inner = O v (256 threads a row), and, in workgroups of their own,
 //                  Obar . v and the previous iteration's x update and convergence test;
-//   mr_colsum_partial   the row-chunk sums of O^T inner;
+//   mr_colsum_rows the row-chunk sums of O^T inner;
 //   mr_form_y_narrow    the chunk sums added up, and y;
 //   mr_finish      alfa, the orthogonalised y, ||y||, the Givens rotation (one workgroup).
 // A launch costs 2 - 3 us whatever it does, so the count of launches bounds small and
 // medium problems: a solve of 2900 samples and 2160 parameters, 100 iterations launched and
-// a third of them made, takes 2.2 ms, of 516 and 480 1.4 ms (15 launches: 4.6 to 6.2 and 6.0;
-// the same bits).  Above kNarrowNp the length-Np work takes the whole chip, in 15
+// a third of them made, takes 1.7 ms, of 516 and 480 1.4 ms (15 launches: 4.6 to 6.2 and 6.0;
+// the same bits); an iteration that is made 30 us (rows 10.7, column sums 10.1, y 4.9, finish
+// 4.5).  Above kNarrowNp the length-Np work takes the whole chip, in 15
 // launches: one workgroup would walk 53 MB an iteration at 2.2 M parameters.
 #include <hip/hip_runtime.h>
 
@@ -57,11 +58,11 @@ enum {
   S_EMEAN, S_EVAR, S_STOP, S_ZERO = 31, S_COUNT = 32
 };
 
+// row-chunk sums of O and of O^T w
 __global__ void __launch_bounds__(256)
     mr_colsum_partial(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo,
-                      int64_t rows, const double *__restrict__ w, const double *__restrict__ w2,
-                      double *partial, double *partial2, const double *skip) {
-  if (skip[0] != 0.0) return;
+                      int64_t rows, const double *__restrict__ w, double *partial,
+                      double *partial2) {
   const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= Np) return;
   const int64_t r0 = (int64_t)blockIdx.y * rows;
@@ -70,11 +71,48 @@ __global__ void __launch_bounds__(256)
   for (int64_t s = r0; s < r1; ++s) {
     const double v = o_dtype == 0 ? ((const double *)O)[s * ldo + p]
                                   : (double)((const float *)O)[s * ldo + p];
-    a.add(w ? v * w[s] : v);
-    if (w2) b.add(v * w2[s]);
+    a.add(v);
+    b.add(v * w[s]);
   }
   partial[(int64_t)blockIdx.y * Np + p] = a.s + a.c;
-  if (w2) partial2[(int64_t)blockIdx.y * Np + p] = b.s + b.c;
+  partial2[(int64_t)blockIdx.y * Np + p] = b.s + b.c;
+}
+
+// a += the products of K rows of O with w, in order; the K loads in flight together
+template <int K, typename T>
+__device__ __forceinline__ void mr_add_rows(const T *O, int64_t ldo, const double *w, Neu2 &a) {
+  T v[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) v[k] = O[k * ldo];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+#pragma clang fp contract(off)
+    const double x = (double)v[k] * w[k];   // rounded: not fused with the sum
+    a.add(x);
+  }
+}
+
+// The row-chunk sums of O^T w of an iteration, over the same chunks in row order.  Bound by the
+// latency of a thread's chain of Ns / kRowChunks loads: 2900 samples, 2160 parameters 22 us with
+// one row at a time, 10 us with eight.
+template <typename T>
+__global__ void __launch_bounds__(256)
+    mr_colsum_rows(int64_t Ns, int64_t Np, const T *__restrict__ O, int64_t ldo, int64_t rows,
+                   const double *__restrict__ w, double *__restrict__ partial,
+                   const double *skip) {
+  if (skip[0] != 0.0) return;
+  const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= Np) return;
+  int64_t s = (int64_t)blockIdx.y * rows;
+  const int64_t r1 = (s + rows < Ns) ? s + rows : Ns;
+  Neu2 a;
+  for (; s + 8 <= r1; s += 8) mr_add_rows<8>(O + s * ldo + p, ldo, w + s, a);
+  if (s + 4 <= r1) {
+    mr_add_rows<4>(O + s * ldo + p, ldo, w + s, a);
+    s += 4;
+  }
+  for (; s < r1; ++s) mr_add_rows<1>(O + s * ldo + p, ldo, w + s, a);
+  partial[(int64_t)blockIdx.y * Np + p] = a.s + a.c;
 }
 
 __global__ void __launch_bounds__(256)
@@ -518,8 +556,7 @@ int sr_minres(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo, c
   hipLaunchKernelGGL(mr_energy, dim3(1), dim3(1024), 0, st, Ns, E, energy_mean, use_given, wE,
                      sc);
   hipLaunchKernelGGL(mr_colsum_partial, dim3(gn, kRowChunks), dim3(256), 0, st, Ns, Np, O,
-                     o_dtype, ldo, rows, (const double *)nullptr, (const double *)wE, partial,
-                     partial2, always);
+                     o_dtype, ldo, rows, (const double *)wE, partial, partial2);
   hipLaunchKernelGGL(mr_colsum_final, dim3(gn), dim3(256), 0, st, Np, partial,
                      1.0 / (double)Ns, m, always);
   hipLaunchKernelGGL(mr_colsum_final, dim3(gn), dim3(256), 0, st, Np, partial2,
@@ -540,6 +577,16 @@ int sr_minres(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo, c
   hipLaunchKernelGGL(mr_zero, dim3(gn), dim3(256), 0, st, Np, w2);
   hipLaunchKernelGGL(mr_zero, dim3(gn), dim3(256), 0, st, Np, wn);
   VMCX_LAUNCHED();
+  // partial <- row-chunk sums of O^T inner
+  auto colsum = [&](const double *skip) {
+    const dim3 grid(gn, kRowChunks), block(256);
+    if (o_dtype == 0)
+      hipLaunchKernelGGL(mr_colsum_rows<double>, grid, block, 0, st, Ns, Np, (const double *)O,
+                         ldo, rows, inner, partial, skip);
+    else
+      hipLaunchKernelGGL(mr_colsum_rows<float>, grid, block, 0, st, Ns, Np, (const float *)O, ldo,
+                         rows, inner, partial, skip);
+  };
   if (Np <= kNarrowNp) {
     const int n = (int)Np;
     MrVecs q{};
@@ -551,9 +598,7 @@ int sr_minres(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo, c
       q.first = it == 0;
       hipLaunchKernelGGL(mr_rows, dim3((unsigned)((Ns + 3) / 4 + 2)), dim3(1024), 0, st, Ns, n,
                          nbd, O, o_dtype, ldo, q, rtol, inner, sc);
-      hipLaunchKernelGGL(mr_colsum_partial, dim3(gn, kRowChunks), dim3(256), 0, st, Ns, Np, O,
-                         o_dtype, ldo, rows, (const double *)inner, (const double *)nullptr,
-                         partial, partial2, (const double *)(sc + S_STOP));
+      colsum(sc + S_STOP);
       hipLaunchKernelGGL(mr_form_y_narrow, dim3((unsigned)((Np + 63) / 64)), dim3(64), 0, st, n,
                          partial, 1.0 / (double)Ns, m, r1, r2, diag_shift, y, sc);
       hipLaunchKernelGGL(mr_finish, dim3(1), dim3(1024), 0, st, n, nbd, r2, y, sc);
@@ -586,9 +631,7 @@ int sr_minres(int64_t Ns, int64_t Np, const void *O, int o_dtype, int64_t ldo, c
       // S v without S: O v, then O^T (O v) / Ns
       hipLaunchKernelGGL(mr_gemv_rows, dim3((unsigned)Ns), dim3(256), 0, st, Np, O, o_dtype, ldo,
                          v, inner, sc);
-      hipLaunchKernelGGL(mr_colsum_partial, dim3(gn, kRowChunks), dim3(256), 0, st, Ns, Np, O,
-                         o_dtype, ldo, rows, (const double *)inner, (const double *)nullptr,
-                         partial, (double *)nullptr, done);
+      colsum(done);
       hipLaunchKernelGGL(mr_colsum_final, dim3(gn), dim3(256), 0, st, Np, partial,
                          1.0 / (double)Ns, Sx, done);
       dot(m, v, S_MV, done);

@@ -1,6 +1,7 @@
-"""MINRES at the sizes where its matrix pass changes form: columns per thread
-(multiples of 1024 columns), two rows or one at a time, the last row alone,
-fewer rows than chunks, and rows too wide for one read (Np > 8192).
+"""MINRES at the sizes where its launches change: strides of 256 columns, one to four
+first-stage blocks of a dot (2048 columns each), four rows a workgroup and the last of them
+alone, fewer rows than chunks, and rows beyond the short form's widest (Np > 8192).  A few
+iterations against the oracle; the updates of whole solves are in test_minres_sums_gpu.py.
 
 Tolerance: four iterations amplify the FP64 rounding of sums over Np terms by
 the ratio of the Krylov vectors' scales, about 1e3 here: 1e3 * 2^-53 *

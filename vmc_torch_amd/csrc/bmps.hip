@@ -1137,7 +1137,7 @@ __global__ void __launch_bounds__(BT, NB == 32 ? 4 : 1)
 // four waves idle in the eigensolver, read two LDS operands per multiply-add in the
 // products and did four times as many (the zero blocks).  LDS 12 KB: up to 13 waves on a
 // CU instead of 4 sides.  6x6 D = 4 chi = 8, 1024 walkers: sampling phase 133.8 ->
-// 48.4 ms (with the join below; 52.6 and 60.1 ms when held to 168 and 128 registers).
+// 47.2 ms (with the join below; some 8 and 24 % more when held to 168 and 128 registers).
 constexpr int BWL = 17;   // LDS row stride of the 16 x 16 blocks
 
 bool bm_wave_fits(int D, int cb) {
